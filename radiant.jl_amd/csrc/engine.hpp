@@ -198,7 +198,7 @@ private:
     double* d_y = nullptr;
 
     // passes
-    void pass_faithful(int g, int prec, int mode, const double* zin, double* zout);
+    void pass_faithful(int g, int prec, int mode, const double* zin, double* zout, const double* caller_q = nullptr);
     void pass_reduced(int g, int prec, int mode, const double* zin, double* zout, void* psi = nullptr);
     void pass_reconstruct(int g, const double* zin_reduced);
     void desc_reduced(PassDesc& pd, int g, int prec, int mode, const double* zin, double* zout);

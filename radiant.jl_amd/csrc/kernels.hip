@@ -296,12 +296,15 @@ __device__ inline short f2bf(float x) {
 // ------------------------------------------------------------------------------------------
 __device__ __align__(256) double g_zero[64];  // zero-initialised, never written
 
-template <typename T, int RT, int CT, typename V>
+// UL: zin and out are in the caller's layout (PassDesc::ul_np moments per column); zin may then be
+// out itself (every element is read and written by one lane, the store depending on the load).
+template <typename T, int RT, int CT, bool UL = false, typename V>
 __device__ inline void epilogue_dgemm(const PassDesc& d, const V (&acc)[RT][CT], int c0, int r0, int li, int lane,
                                       int M, int Nc) {
     const bool hasz = d.zin != nullptr;
     const double* __restrict__ zb = hasz ? d.zin : g_zero;
-    const size_t zrs = hasz ? (size_t)Nc : 0;
+    const size_t zrs = hasz ? (UL ? (size_t)1 : (size_t)Nc) : 0;
+    const size_t cs = UL ? (size_t)d.ul_np : (size_t)1, rs = UL ? (size_t)1 : (size_t)Nc;
     const double zs = hasz ? 1.0 : 0.0, sg = hasz ? -1.0 : 1.0;
     // one row tile at a time (the zin values of a whole wave tile would hold 2*RT*CT*4 VGPRs
     // and halve the waves a SIMD can hold); the loads of tile t + 1 are issued before the
@@ -314,7 +317,7 @@ __device__ inline void epilogue_dgemm(const PassDesc& d, const V (&acc)[RT][CT],
             for (int r = 0; r < 4; ++r) {
                 const int col = c0 + 16 * u + li, row = r0 + 16 * t + acc_row<T>(lane, r);
                 const int cc = col < Nc ? col : Nc - 1, rc = row < M ? row : M - 1;
-                zt[u][r] = gld(zb + (size_t)rc * zrs + (hasz ? cc : li));
+                zt[u][r] = gld(zb + (size_t)rc * zrs + (hasz ? cc * cs : (size_t)li));
             }
     };
     zload(0, z[0]);
@@ -327,12 +330,12 @@ __device__ inline void epilogue_dgemm(const PassDesc& d, const V (&acc)[RT][CT],
             for (int r = 0; r < 4; ++r) {
                 const int col = c0 + 16 * u + li, row = r0 + 16 * t + acc_row<T>(lane, r);
                 const double v = zs * z[t & 1][u][r] + sg * (double)acc[t][u][r];
-                if (col < Nc && row < M) gst(d.out + (size_t)row * Nc + col, v);
+                if (col < Nc && row < M) gst(d.out + row * rs + col * cs, v);
             }
     }
 }
 
-template <typename T, int RT, int CT, bool MG, int NS, bool ADD = false>
+template <typename T, int RT, int CT, bool MG, int NS, bool ADD = false, bool UL = false>
 __device__ __forceinline__ void contract_body(const PassDesc& d, const GemmTask tk, int* rows_s) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int Nc = d.Nc;
@@ -371,13 +374,16 @@ __device__ __forceinline__ void contract_body(const PassDesc& d, const GemmTask 
     if (MG) {
         const int* __restrict__ rows = d.phi_rows;
         for (int i = threadIdx.x; i < K; i += blockDim.x) rows_s[i] = rows ? rows[i] : i;
-        if (hasq) { qb = qlout; qks = (size_t)Nc; }
-        if (hasp) { pb = phi_in; pks = (size_t)Nc; wb = sigw; wks = 1; }
+        // caller layout: a moment is the row map's entry (the operator rows' own moments), a column
+        // ul_np values on
+        if (hasq) { qb = qlout; qks = UL ? (size_t)1 : (size_t)Nc; }
+        if (hasp) { pb = phi_in; pks = UL ? (size_t)1 : (size_t)Nc; wb = sigw; wks = 1; }
+        const int cs = UL ? d.ul_np : 1;
 #pragma unroll
         for (int u = 0; u < CT; ++u) {
             const int mc = gld(d.mat + colc[u]);
-            qcol[u] = hasq ? colc[u] : li;
-            pcol[u] = hasp ? colc[u] : li;
+            qcol[u] = hasq ? colc[u] * cs : li;
+            pcol[u] = hasp ? colc[u] * cs : li;
             wrow[u] = hasp ? mc * K : li;
         }
         __syncthreads();
@@ -400,7 +406,7 @@ __device__ __forceinline__ void contract_body(const PassDesc& d, const GemmTask 
 #pragma unroll
         for (int u = 0; u < CT; ++u) {
             if (MG) {
-                g.q[u] = gld(qb + kc * qks + qcol[u]);
+                g.q[u] = gld(qb + (UL ? rows_s[kc] : kc) * qks + qcol[u]);
                 g.w[u] = gld(wb + kc * wks + wrow[u]);
                 g.p[u] = gld(pb + (size_t)rows_s[kc] * pks + pcol[u]);
             } else {
@@ -456,15 +462,15 @@ __device__ __forceinline__ void contract_body(const PassDesc& d, const GemmTask 
     } else {
         // out = zin - D psi (I - A matvec) or D psi: every zin value is loaded before the first
         // store, unconditionally, and combined as zs*z + sg*v (a select would branch the loads).
-        epilogue_dgemm<T, RT, CT>(d, acc, c0, r0, li, lane, M, Nc);
+        epilogue_dgemm<T, RT, CT, UL>(d, acc, c0, r0, li, lane, M, Nc);
     }
 }
 
-template <typename T, int RT, int CT, bool MG, int NS, bool ADD = false>
+template <typename T, int RT, int CT, bool MG, int NS, bool ADD = false, bool UL = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((sizeof(T) == 4 && !MG) ? 3 : 2))) void contract_kernel(const PassDesc* __restrict__ pds, const GemmTask* __restrict__ tasks) {
     __shared__ int rows_s[MG ? CONTRACT_KMAX : 1];
     const GemmTask tk = tasks[blockIdx.x];
-    contract_body<T, RT, CT, MG, NS, ADD>(pds[tk.prob], tk, rows_s);
+    contract_body<T, RT, CT, MG, NS, ADD, UL>(pds[tk.prob], tk, rows_s);
 }
 
 // FP64 and FP32 passes of different problems in one launch (PassDesc::prec per workgroup).
@@ -2778,6 +2784,18 @@ void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, h
     if (v == 0) launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, false, 4, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     else launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, false, 2, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     tune_commit(t);
+    RT_HIP(hipGetLastError());
+}
+
+// The caller-layout forms take the default pipeline depths (this call times nothing).
+void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+    if (ntasks <= 0) return;
+    launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, true, 2, false, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+    RT_HIP(hipGetLastError());
+}
+void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+    if (ntasks <= 0) return;
+    launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, false, 4, false, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     RT_HIP(hipGetLastError());
 }
 

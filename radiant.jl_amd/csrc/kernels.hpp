@@ -102,6 +102,9 @@ struct PassDesc {
     // of tagged 64-bit words, both zero before the first launch
     unsigned long long* sclaim;
     unsigned long long* shand;
+    // Caller layout of the allocation-free pass (launch_mgemm_caller, launch_dgemm_caller): qlout,
+    // phi_in, zin and out hold ul_np moments per column, moment fastest, as Radiant's state does.
+    int ul_np;
 };
 
 enum Prec { P64 = 0, P32 = 1, PBF16 = 2,
@@ -132,6 +135,9 @@ int sweep_pencils_per_thread(int P);
 size_t sweep_lds_bytes(int prec, int Nx, int Ny, int Nz, int Nmat, int nbuf);
 
 void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
+// The FP64 contractions of one problem on states in the caller's layout (PassDesc::ul_np)
+void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
+void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
 // FP64 D contraction of (psi + psi_add), one problem (PassDesc::psi_add non-null)
 void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
 void launch_sweep(int prec, const PassDesc* d_pd, const SweepTask* tasks, int ntasks, int ppt, int nbuf,
