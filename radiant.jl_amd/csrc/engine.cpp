@@ -589,6 +589,16 @@ Problem::Problem(const rt_problem_desc& d, hipStream_t stream) {
         d_mg = gemm_tasks(Nd, n_mg);
         d_dgf = gemm_tasks(Np, n_dgf);
         d_dga = gemm_tasks(Nact, n_dga);
+        if (state_mode == RT_STATE_FAITHFUL || has_bc) {
+            std::vector<BndTask> t;
+            for (int ax = 0; ax < ndims; ++ax)
+                for (int f = 0; f < 2; ++f)
+                    for (int i = 0; i < ceil_div((int)npos[ax], BND_CELLS); ++i)
+                        for (int r = 0; r < ceil_div(Nps, BND_ROWS); ++r) t.push_back({2 * ax + f, r, i, 0});
+            n_bnd = (int)t.size();
+            d_bnd = dalloc<BndTask>(std::max<size_t>(1, t.size()));
+            if (n_bnd) upload(d_bnd, t, st);
+        }
         std::vector<SweepTask> sw(Nd);
         for (int n = 0; n < Nd; ++n) sw[n] = {0, n};
         d_sw = dalloc<SweepTask>(Nd); upload(d_sw, sw, st);
@@ -794,9 +804,21 @@ void Problem::launch_pass(PassDesc& pd, int prec, bool full_rows) {
     const bool emsrc = em && pd.phi_in;
     const double* em_qin = pd.qlout;
     if (emsrc) pd.qlout = d_emq;
-    k_set_pd(pd, d_pd, st);
-    if (pd.bin_x) launch_bndin(d_pd, (int)bin_total, st);  // incoming fluxes of non-void faces
-    if (fpsrc) launch_fp_source(d_pd, (long)Nact * Nc, st);
+    // the pass's first kernel takes the PassDesc by value and stores it for the others
+    bool have_pd = false;
+    if (pd.bin_x && bin_total > 0) {  // incoming fluxes of non-void faces
+        launch_bndin_first(pd, d_pd, (int)bin_total, st);
+        have_pd = true;
+    }
+    if (fpsrc) {
+        if (have_pd) launch_fp_source(d_pd, (long)Nact * Nc, st);
+        else launch_fp_source_first(pd, d_pd, (long)Nact * Nc, st);
+        have_pd = true;
+    }
+    if (!have_pd && prec == PBF16) {
+        k_set_pd(pd, d_pd, st);
+        have_pd = true;
+    }
     if (emsrc) launch_em_source(pd.phi_in, pd.phi_rows, d_emM + (size_t)em_g * Nact * Nact, em_qin, d_emq, Nact, Nc, st);
     auto timed = [&](int kernel, auto&& fn) {
         if (!profiling) {
@@ -812,7 +834,9 @@ void Problem::launch_pass(PassDesc& pd, int prec, bool full_rows) {
     };
     const bool caller = pd.ul_np > 0;
     timed(0, [&] {
-        if (caller) launch_mgemm_caller(d_pd, d_mg, n_mg, st);
+        const PassDesc* first = have_pd ? nullptr : &pd;
+        if (caller) launch_mgemm_caller(d_pd, d_mg, n_mg, st, first);
+        else if (first) launch_mgemm_first(prec, pd, d_pd, d_mg, n_mg, st);
         else launch_mgemm(prec, d_pd, d_mg, n_mg, st);
     });
     if (pd.psiE_in && !bfp) launch_csd_source(d_pd, (long)Nd * Nc, st);  // energy inflow (FP64 passes)
@@ -850,11 +874,15 @@ void Problem::launch_pass(PassDesc& pd, int prec, bool full_rows) {
             launch_sweep(sp, d_pd, d_sw, Nd, sw_ppt, sw_nbuf[prec], sw_block, sw_lds[prec], st);
     });
     if (pd.psiE_out && !bfp) launch_csd_out(d_pd, (long)Nd * Nc, st);
+    // FP64 exit-face moments ride in the D contraction's launch; on their own where the kernels are
+    // timed one by one
+    const bool merged = pd.bout_x && prec == P64 && !profiling;
     timed(2, [&] {
-        if (caller) launch_dgemm_caller(d_pd, d_dgf, n_dgf, st);
+        if (caller) launch_dgemm_caller(d_pd, d_dgf, n_dgf, d_bnd, merged ? n_bnd : 0, st);
+        else if (merged) launch_dgemm_bnd(d_pd, full_rows ? d_dgf : d_dga, full_rows ? n_dgf : n_dga, d_bnd, n_bnd, st);
         else launch_dgemm(prec, d_pd, full_rows ? d_dgf : d_dga, full_rows ? n_dgf : n_dga, st);
     });
-    if (pd.bout_x) timed(3, [&] { launch_bndmom(d_pd, 1, (int)nb, st); });
+    if (pd.bout_x && !merged) timed(3, [&] { launch_bndmom(d_pd, 1, (int)nb, st); });
     counters.passes += 1;
     if (prec != P64) counters.passes_lo += 1;
     counters.updates_raw += (double)Ncell * Nd;

@@ -178,6 +178,8 @@ private:
     PassDesc* d_pd = nullptr;
     GemmTask *d_mg = nullptr, *d_dgf = nullptr, *d_dga = nullptr;
     int n_mg = 0, n_dgf = 0, n_dga = 0;
+    BndTask* d_bnd = nullptr;  // exit-face moment tasks of the D contraction's launch
+    int n_bnd = 0;
     SweepTask* d_sw = nullptr;
     int sw_ppt = 1, sw_block = 64, sw_nbuf[3] = {2, 2, 2};
     int rows_per_lane = -1;   // > 0: 1D/2D wave-per-direction sweep

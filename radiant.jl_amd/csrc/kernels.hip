@@ -473,6 +473,116 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((sizeof(T) 
     contract_body<T, RT, CT, MG, NS, ADD, UL>(pds[tk.prob], tk, rows_s);
 }
 
+// The PassDesc of a single problem travels as the argument of the pass's first kernel, which stores
+// it for the later ones: a launch of its own to write it (4 us, most of them latency) is saved.  The
+// copy reads the argument segment by word, as a dynamic index into the argument itself would move
+// it to scratch; the PassDesc is the first argument, at offset 0.
+__device__ inline void store_pd(PassDesc* dst) {
+    static_assert(sizeof(PassDesc) % 8 == 0, "PassDesc is copied by 64-bit words");
+    const unsigned long long* src = (const unsigned long long*)__builtin_amdgcn_kernarg_segment_ptr();
+    for (int i = threadIdx.x; i < (int)(sizeof(PassDesc) / 8); i += blockDim.x) ((unsigned long long*)dst)[i] = src[i];
+}
+template <typename T, int RT, int CT, int NS, bool UL = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void contract_first_kernel(
+    const PassDesc v, PassDesc* dst, const GemmTask* __restrict__ tasks) {
+    __shared__ int rows_s[CONTRACT_KMAX];
+    if (blockIdx.x == 0) store_pd(dst);
+    contract_body<T, RT, CT, true, NS, false, UL>(v, tasks[blockIdx.x], rows_s);
+}
+
+// Half-range moments of an exit face (see bndmom_kernel) as a contraction over the directions that
+// leave through it, on the FP64 matrix cores: 32 moments x 128 face positions per workgroup, 32 x 32
+// per wave.  It runs as extra workgroups of the D contraction's launch, which it neither reads from
+// nor writes to.  One thread per moment and position, in a launch of its own, took 10 us (2D, 128 x 128,
+// 128 directions) and 22 us (3D, 40 x 37 x 42, 80 directions); with the PassDesc launch gone too a
+// pass of the first went from 115 to 101 us, of a 31 x 29 x 30 box from 130 to 113 us.
+__device__ __forceinline__ void bnd_body(const PassDesc& d, const BndTask tk) {
+    constexpr int RT = 2, CT = 2, NS = 4;
+    const int ax = tk.code >> 1, f = tk.code & 1;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kk = lane >> 4, li = lane & 15;
+    const int fm_ = ax == 0 ? d.fm_x : (ax == 1 ? d.fm_y : d.fm_z), fm = fm_ > 1 ? fm_ : 1;
+    const int N = (ax == 0 ? d.Ny * d.Nz : (ax == 1 ? d.Nx * d.Nz : d.Nx * d.Ny)) * fm;
+    const int M = d.Nps, K = d.excnt[ax][f];
+    const double* __restrict__ A = ax == 0 ? d.Dexit_x : (ax == 1 ? d.Dexit_y : d.Dexit_z);
+    const double* __restrict__ B = (const double*)(ax == 0 ? d.bx : (ax == 1 ? d.by : d.bz));
+    const int* __restrict__ lst = (ax == 0 ? d.exlist_x : (ax == 1 ? d.exlist_y : d.exlist_z)) + f * d.Nd;
+    double* out = ax == 0 ? d.bout_x : (ax == 1 ? d.bout_y : d.bout_z);
+    const double* zin = ax == 0 ? d.bzin_x : (ax == 1 ? d.bzin_y : d.bzin_z);
+    const int c0 = tk.tile * BND_CELLS + wave * (CT * 16), r0 = tk.rgroup * BND_ROWS;
+    int colc[CT], rowc[RT];
+#pragma unroll
+    for (int u = 0; u < CT; ++u) colc[u] = c0 + 16 * u + li < N ? c0 + 16 * u + li : N - 1;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) rowc[t] = r0 + 16 * t + li < M ? r0 + 16 * t + li : M - 1;
+    v4d acc[RT][CT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int u = 0; u < CT; ++u) acc[t][u] = (v4d)(0.0);
+    struct Stage { double a[RT], b[CT]; };
+    auto index = [&](int s) {
+        const int k = 4 * s + kk;
+        return gld(lst + (k < K ? k : K - 1));
+    };
+    auto load = [&](int n, Stage& g) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t) g.a[t] = gld(A + (size_t)n * M + rowc[t]);
+#pragma unroll
+        for (int u = 0; u < CT; ++u) g.b[u] = gld(B + (size_t)n * N + colc[u]);
+    };
+    // padding (k past the list) is zeroed by a factor on the operator; rows and cells past the end
+    // repeat the last one and are not stored
+    auto mma = [&](int s, const Stage& g) {
+        const double ok = 4 * s + kk < K ? 1.0 : 0.0;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const double a = g.a[t] * ok;
+#pragma unroll
+            for (int u = 0; u < CT; ++u) acc[t][u] = mfma4(a, ok != 0.0 ? g.b[u] : 0.0, acc[t][u]);
+        }
+    };
+    const int nsteps = (K + 3) >> 2;
+    if (K > 0) {
+        Stage g[NS];
+        int nx[NS];  // directions of the steps whose operands are loaded next
+#pragma unroll
+        for (int i = 0; i < NS; ++i) nx[i] = index(i);
+#pragma unroll
+        for (int i = 0; i < NS - 1; ++i) load(nx[i], g[i]);
+        for (int s = 0; s < nsteps; s += NS) {
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                const int j = (i + NS - 1) % NS;  // step s + i + NS - 1
+                __builtin_amdgcn_sched_barrier(0);
+                load(nx[j], g[j]);
+                nx[i] = index(s + i + NS);
+                __builtin_amdgcn_sched_barrier(0);
+                if (s + i < nsteps) mma(s + i, g[i]);  // wave-uniform
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int u = 0; u < CT; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int col = c0 + 16 * u + li, row = r0 + 16 * t + acc_row<double>(lane, r);
+                if (col >= N || row >= M) continue;
+                const int pos = col / fm, m = col - pos * fm;
+                const size_t j = row + (size_t)M * (m + (size_t)fm * (f + 2 * (size_t)pos));
+                gst(out + j, zin ? gld(zin + j) - acc[t][u][r] : acc[t][u][r]);
+            }
+}
+template <int RT, int CT, int NS, bool UL = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void contract_bnd_kernel(
+    const PassDesc* __restrict__ pds, const GemmTask* __restrict__ tasks, int ntasks,
+    const BndTask* __restrict__ btasks) {
+    __shared__ int rows_s[1];
+    if ((int)blockIdx.x < ntasks) contract_body<double, RT, CT, false, NS, false, UL>(pds[0], tasks[blockIdx.x], rows_s);
+    else bnd_body(pds[0], btasks[blockIdx.x - ntasks]);
+}
+
 // FP64 and FP32 passes of different problems in one launch (PassDesc::prec per workgroup).
 template <int RT, int CT, bool MG, int NS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void contract_mixed_kernel(const PassDesc* __restrict__ pds,
@@ -2051,8 +2161,7 @@ __global__ __launch_bounds__(256) void bndmom_kernel(const PassDesc* __restrict_
 // periodic), each summed in moment order.
 // One thread per (axis, direction, position).
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void bndin_kernel(const PassDesc* __restrict__ pds) {
-    const PassDesc& d = pds[0];
+__device__ __forceinline__ void bndin_body(const PassDesc& d) {
     const int Nd = d.Nd, Nps = d.Nps;
     // positions times face moments per axis (the moments of a general 2D closure; 1 otherwise)
     const int fm[3] = {d.fm_x > 1 ? d.fm_x : 1, d.fm_y > 1 ? d.fm_y : 1, d.fm_z > 1 ? d.fm_z : 1};
@@ -2085,6 +2194,11 @@ __global__ __launch_bounds__(256) void bndin_kernel(const PassDesc* __restrict__
         out[j] = v;
     }
 }
+__global__ __launch_bounds__(256) void bndin_kernel(const PassDesc* __restrict__ pds) { bndin_body(pds[0]); }
+__global__ __launch_bounds__(256) void bndin_first_kernel(const PassDesc v, PassDesc* dst) {
+    if (blockIdx.x == 0) store_pd(dst);
+    bndin_body(v);
+}
 
 // ------------------------------------------------------------------------------------------
 // Continuous slowing down with the DD scheme of order 1 in energy (flux_{1,2,3}D_BFP of
@@ -2110,8 +2224,7 @@ __global__ __launch_bounds__(256) void csd_out_kernel(const PassDesc* __restrict
 
 // Angular Fokker-Planck source (fokker_planck_source.jl:26-36) added to the out-of-group source
 // before the moment -> direction contraction: one thread per (moment k, cell c), cells fastest.
-__global__ __launch_bounds__(256) void fp_source_kernel(const PassDesc* __restrict__ pds, long n) {
-    const PassDesc& d = pds[0];
+__device__ __forceinline__ void fp_source_body(const PassDesc& d, long n) {
     const int K = d.Nact, Nc = d.Nc;
     const int* __restrict__ rows = d.phi_rows;
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
@@ -2121,6 +2234,11 @@ __global__ __launch_bounds__(256) void fp_source_kernel(const PassDesc* __restri
         for (int j = 0; j < K; ++j) s += Mk[j] * d.phi_in[(size_t)(rows ? rows[j] : j) * Nc + c];
         d.fpq[i] = (d.fp_qin ? d.fp_qin[i] : 0.0) + d.fpT[d.mat[c]] * s;
     }
+}
+__global__ __launch_bounds__(256) void fp_source_kernel(const PassDesc* __restrict__ pds, long n) { fp_source_body(pds[0], n); }
+__global__ __launch_bounds__(256) void fp_source_first_kernel(const PassDesc v, PassDesc* dst, long n) {
+    if (blockIdx.x == 0) store_pd(dst);
+    fp_source_body(v, n);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2758,10 +2876,15 @@ static void contract_launch(int prec, const PassDesc* d_pd, const GemmTask* task
     else if (prec == P64) launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, MG, NS>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     else launch_timed(contract_kernel<float, GEMM_RT, GEMM_CT, MG, NS>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
 }
+template <int NS>
+static void contract_first(int prec, const PassDesc& pd, PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+    if (prec == P64) launch_timed(contract_first_kernel<double, GEMM_RT, GEMM_CT, NS>, dim3(ntasks), dim3(256), 0, st, pd, d_pd, tasks);
+    else launch_timed(contract_first_kernel<float, GEMM_RT, GEMM_CT, NS>, dim3(ntasks), dim3(256), 0, st, pd, d_pd, tasks);
+}
 
 // Pipeline depth (k steps in flight) of the contractions: the default first, then the autotuner's
 // alternative (same accumulation order, so the same bits); BF16 operands keep their one shape.
-void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+static void mgemm_any(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, const PassDesc* first) {
     if (ntasks <= 0) return;
     if (prec == PBF16) {
         launch_timed(contract_bf16_kernel<GEMM_RT, GEMM_CT, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
@@ -2769,11 +2892,22 @@ void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int nta
         TuneTicket t;
         const int v = tune_choose({prec, 2, 0, 0, 0, ilog2(ntasks)}, 2, t);
         if (t.a) set_launch_events(t.a, t.b);
-        if (v == 0) contract_launch<true, 2>(prec, d_pd, tasks, ntasks, st);
+        if (first) {
+            if (v == 0) contract_first<2>(prec, *first, const_cast<PassDesc*>(d_pd), tasks, ntasks, st);
+            else contract_first<3>(prec, *first, const_cast<PassDesc*>(d_pd), tasks, ntasks, st);
+        } else if (v == 0) contract_launch<true, 2>(prec, d_pd, tasks, ntasks, st);
         else contract_launch<true, 3>(prec, d_pd, tasks, ntasks, st);
         tune_commit(t);
     }
     RT_HIP(hipGetLastError());
+}
+
+void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+    mgemm_any(prec, d_pd, tasks, ntasks, st, nullptr);
+}
+void launch_mgemm_first(int prec, const PassDesc& pd, PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+    if (prec != P64 && prec != P32) throw std::runtime_error("launch_mgemm_first: FP64 and FP32 passes only");
+    mgemm_any(prec, d_pd, tasks, ntasks, st, &pd);
 }
 
 void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
@@ -2788,14 +2922,30 @@ void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, h
 }
 
 // The caller-layout forms take the default pipeline depths (this call times nothing).
-void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, const PassDesc* first) {
     if (ntasks <= 0) return;
-    launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, true, 2, false, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+    if (first)
+        launch_timed(contract_first_kernel<double, GEMM_RT, GEMM_CT, 2, true>, dim3(ntasks), dim3(256), 0, st, *first,
+                     const_cast<PassDesc*>(d_pd), tasks);
+    else
+        launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, true, 2, false, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     RT_HIP(hipGetLastError());
 }
-void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt,
+                         hipStream_t st) {
     if (ntasks <= 0) return;
-    launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, false, 4, false, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+    launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 4, true>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
+    RT_HIP(hipGetLastError());
+}
+
+void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt, hipStream_t st) {
+    if (ntasks <= 0) return;
+    TuneTicket t;
+    const int v = tune_choose({P64, 3, 0, 0, 1, ilog2(ntasks)}, 2, t);
+    if (t.a) set_launch_events(t.a, t.b);
+    if (v == 0) launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 4>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
+    else launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 2>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
+    tune_commit(t);
     RT_HIP(hipGetLastError());
 }
 
@@ -3456,6 +3606,15 @@ void launch_sweep_1d_ho(int prec, const PassDesc* d_pd, int Nd, int K, hipStream
 
 void launch_fp_source(const PassDesc* d_pd, long n, hipStream_t st) {
     hipLaunchKernelGGL(fp_source_kernel, dim3(grid_for((size_t)n)), dim3(256), 0, st, d_pd, n);
+    RT_HIP(hipGetLastError());
+}
+
+void launch_bndin_first(const PassDesc& pd, PassDesc* d_pd, int total, hipStream_t st) {
+    hipLaunchKernelGGL(bndin_first_kernel, dim3(grid_for((size_t)total)), dim3(256), 0, st, pd, d_pd);
+    RT_HIP(hipGetLastError());
+}
+void launch_fp_source_first(const PassDesc& pd, PassDesc* d_pd, long n, hipStream_t st) {
+    hipLaunchKernelGGL(fp_source_first_kernel, dim3(grid_for((size_t)n)), dim3(256), 0, st, pd, d_pd, n);
     RT_HIP(hipGetLastError());
 }
 

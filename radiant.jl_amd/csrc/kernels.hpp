@@ -134,10 +134,25 @@ struct SweepTask { int prob, dir; };
 int sweep_pencils_per_thread(int P);
 size_t sweep_lds_bytes(int prec, int Nx, int Ny, int Nz, int Nmat, int nbuf);
 
+// _first: the launch takes the PassDesc by value and stores it in d_pd for the launches that follow it
+// on the stream (single problems, FP64 and FP32).
+void launch_mgemm_first(int prec, const PassDesc& pd, PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
 void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
+// The same for the kernels that come before the contraction.
+void launch_bndin_first(const PassDesc& pd, PassDesc* d_pd, int total, hipStream_t st);
+void launch_fp_source_first(const PassDesc& pd, PassDesc* d_pd, long n, hipStream_t st);
+// FP64 D contraction of one problem with the half-range moments of its exit faces (nbt boundary
+// tasks, as a pass with PassDesc::bout_* wants them) in one launch.
+struct BndTask { int code, rgroup, tile, pad; };  // code: 2 * axis + face
+constexpr int BND_ROWS = 32;    // half-range moments per boundary task
+constexpr int BND_CELLS = 128;  // face positions (times face moments) per boundary task
+void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt,
+                      hipStream_t st);
 // The FP64 contractions of one problem on states in the caller's layout (PassDesc::ul_np)
-void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
-void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
+void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st,
+                         const PassDesc* first);
+void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt,
+                         hipStream_t st);
 // FP64 D contraction of (psi + psi_add), one problem (PassDesc::psi_add non-null)
 void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
 void launch_sweep(int prec, const PassDesc* d_pd, const SweepTask* tasks, int ntasks, int ppt, int nbuf,

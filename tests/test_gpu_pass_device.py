@@ -35,7 +35,7 @@ def _problem(form):
 
 @pytest.mark.parametrize("form", ["slab1", "slab257", "plane72", "box48", "reflected", "closure", "fokker-planck"])
 def test_caller_layout_forms(form):
-    import torch
+    from test_zz_no_alloc import _Dev
     from radiant_hip import _lib, solver
     p = _problem(form)
     h = solver.ResidentProblem(p)
@@ -44,22 +44,18 @@ def test_caller_layout_forms(form):
         rng = np.random.default_rng(40)
         z = rng.uniform(-1.0, 1.0, S)
         q = rng.uniform(0.0, 1.0, (d.Nc, d.Np)) * (np.asarray(d.ang.pl)[None] <= p.Lxs)
-        dz, dq = torch.from_numpy(z).cuda(), torch.from_numpy(q.ravel()).cuda()
+        dev = _Dev()
+        dq = dev.put(q.ravel())
         for g in range(p.G):
             for mode in (0, 1, 2):
                 print(form, g, mode, flush=True)
                 want = h.transport_pass(g, mode, q.ravel(), z)
-                out = torch.empty_like(dz)
-                same = dz.clone()
-                buf = torch.empty(S + 3, device="cuda", dtype=torch.float64)
-                buf[:S] = dz
-                torch.cuda.synchronize()
-                call = lambda i, o: _lib.check(_lib.lib().rt_problem_pass_device(
-                    h.h, g, mode, C.c_void_p(dq.data_ptr()), C.c_void_p(i.data_ptr()), C.c_void_p(o.data_ptr())))
-                call(dz, out)
-                call(same, same)          # in place
-                call(buf[:S], buf[3:])    # overlapping
-                for got in (out, same, buf[3:]):
-                    assert np.array_equal(got.cpu().numpy(), want), (form, g, mode)
+                for shift in (None, 0, 3):  # beside the input, in place, overlapping it
+                    dz = dev.put(np.concatenate([z, np.zeros(3)]))
+                    out = dev.alloc(S * 8) if shift is None else C.c_void_p(dz.value + 8 * shift)
+                    _lib.check(_lib.lib().rt_problem_pass_device(h.h, g, mode, dq, dz, out))
+                    assert np.array_equal(dev.get(out, S), want), (form, g, mode, shift)
+                    dev.free(*((dz,) if shift is not None else (dz, out)))
+        dev.free(dq)
     finally:
         h.close()
