@@ -535,18 +535,18 @@ void BatchSolver::launch_passes(const std::vector<int>& who, const std::vector<P
         });
         // the split launches of a mixed round: FP64 tasks [0, n64), FP32 tasks [n64, n); the
         // timing events of the pair start at the first launch and stop at the last
-        auto gemm2 = [split](void (*fn)(int, const PassDesc*, const GemmTask*, int, hipStream_t), int prec_,
+        auto gemm2 = [split](void (*fn)(int, const PassDesc*, const GemmTask*, int, hipStream_t, bool), int prec_,
                              const PassDesc* pd, GemmTask* t, int n64, int n, hipStream_t s_) {
             if (!split || n64 == 0 || n64 == n) {
-                fn(split ? (n64 == n ? (int)P64 : (int)P32) : prec_, pd, t, n, s_);
+                fn(split ? (n64 == n ? (int)P64 : (int)P32) : prec_, pd, t, n, s_, false);
                 return;
             }
             hipEvent_t a, b;
             take_launch_events(&a, &b);
             set_launch_events(a, nullptr);
-            fn(P64, pd, t, n64, s_);
+            fn(P64, pd, t, n64, s_, false);
             set_launch_events(nullptr, b);
-            fn(P32, pd, t + n64, n - n64, s_);
+            fn(P32, pd, t + n64, n - n64, s_, false);
             set_launch_events(nullptr, nullptr);
         };
         if (nm)

@@ -573,9 +573,11 @@ Problem::Problem(const rt_problem_desc& d, hipStream_t stream) {
         d_bscratch = dalloc<double>(std::max<size_t>(1, nb));
         d_pd = dalloc<PassDesc>(1);
         // ---- work tables
-        auto gemm_tasks = [&](int rows, int& ntask) {
+        auto gemm_tasks = [&](int rows, int& ntask, bool& small) {
             std::vector<GemmTask> t;
-            const int tiles = ceil_div(Nc, GEMM_CELLS), rg = ceil_div(rows, GEMM_ROWS);
+            small = gemm_small(rows, Nc);
+            const int tiles = ceil_div(Nc, small ? GEMM_SMALL_CELLS : GEMM_CELLS),
+                      rg = ceil_div(rows, small ? GEMM_SMALL_ROWS : GEMM_ROWS);
             for (int i = 0; i < tiles * rg; ++i) {
                 int tile, r;
                 gemm_task_order(i, tiles, rg, tile, r);
@@ -586,9 +588,9 @@ Problem::Problem(const rt_problem_desc& d, hipStream_t stream) {
             upload(p, t, st);
             return p;
         };
-        d_mg = gemm_tasks(Nd, n_mg);
-        d_dgf = gemm_tasks(Np, n_dgf);
-        d_dga = gemm_tasks(Nact, n_dga);
+        d_mg = gemm_tasks(Nd, n_mg, sm_mg);
+        d_dgf = gemm_tasks(Np, n_dgf, sm_dgf);
+        d_dga = gemm_tasks(Nact, n_dga, sm_dga);
         if (state_mode == RT_STATE_FAITHFUL || has_bc) {
             std::vector<BndTask> t;
             for (int ax = 0; ax < ndims; ++ax)
@@ -835,9 +837,9 @@ void Problem::launch_pass(PassDesc& pd, int prec, bool full_rows) {
     const bool caller = pd.ul_np > 0;
     timed(0, [&] {
         const PassDesc* first = have_pd ? nullptr : &pd;
-        if (caller) launch_mgemm_caller(d_pd, d_mg, n_mg, st, first);
-        else if (first) launch_mgemm_first(prec, pd, d_pd, d_mg, n_mg, st);
-        else launch_mgemm(prec, d_pd, d_mg, n_mg, st);
+        if (caller) launch_mgemm_caller(d_pd, d_mg, n_mg, st, first, sm_mg);
+        else if (first) launch_mgemm_first(prec, pd, d_pd, d_mg, n_mg, st, sm_mg);
+        else launch_mgemm(prec, d_pd, d_mg, n_mg, st, sm_mg);
     });
     if (pd.psiE_in && !bfp) launch_csd_source(d_pd, (long)Nd * Nc, st);  // energy inflow (FP64 passes)
     timed(1, [&] {
@@ -878,9 +880,12 @@ void Problem::launch_pass(PassDesc& pd, int prec, bool full_rows) {
     // timed one by one
     const bool merged = pd.bout_x && prec == P64 && !profiling;
     timed(2, [&] {
-        if (caller) launch_dgemm_caller(d_pd, d_dgf, n_dgf, d_bnd, merged ? n_bnd : 0, st);
-        else if (merged) launch_dgemm_bnd(d_pd, full_rows ? d_dgf : d_dga, full_rows ? n_dgf : n_dga, d_bnd, n_bnd, st);
-        else launch_dgemm(prec, d_pd, full_rows ? d_dgf : d_dga, full_rows ? n_dgf : n_dga, st);
+        const GemmTask* dg = full_rows ? d_dgf : d_dga;
+        const int n_dg = full_rows ? n_dgf : n_dga;
+        const bool sm = full_rows ? sm_dgf : sm_dga;
+        if (caller) launch_dgemm_caller(d_pd, dg, n_dg, d_bnd, merged ? n_bnd : 0, st, sm);
+        else if (merged) launch_dgemm_bnd(d_pd, dg, n_dg, d_bnd, n_bnd, st, sm);
+        else launch_dgemm(prec, d_pd, dg, n_dg, st, sm);
     });
     if (pd.bout_x && !merged) timed(3, [&] { launch_bndmom(d_pd, 1, (int)nb, st); });
     counters.passes += 1;
@@ -1041,8 +1046,8 @@ void Problem::reconstruct_sweep_free(int g, const double* zin_reduced, const dou
     }
     counters.passes += 1;  // a pass without sweep
     auto dg = [&] {
-        if (fold) launch_dgemm_add(d_pd, d_dgf, n_dgf, st);
-        else launch_dgemm(P64, d_pd, d_dgf, n_dgf, st);
+        if (fold) launch_dgemm_add(d_pd, d_dgf, n_dgf, st, sm_dgf);
+        else launch_dgemm(P64, d_pd, d_dgf, n_dgf, st, sm_dgf);
     };
     if (profiling) {
         if (ev_next + 2 > 4096) collect_kernel_times();
@@ -1765,9 +1770,9 @@ void test_contraction(int which, int prec, int M, int K, int N, const double* A,
         std::memset(&pd, 0, sizeof(pd));
         pd.Nc = N; pd.Nmat = 1; pd.mat = dmat; pd.sigw = dsig;
         std::vector<GemmTask> t;
-        const int rows = which == 0 ? M : M;
-        for (int r = 0; r < (rows + GEMM_ROWS - 1) / GEMM_ROWS; ++r)
-            for (int i = 0; i < (N + GEMM_CELLS - 1) / GEMM_CELLS; ++i) t.push_back({0, i, r, 0});
+        const bool small = gemm_small(M, N);
+        for (int r = 0; r < ceil_div(M, small ? GEMM_SMALL_ROWS : GEMM_ROWS); ++r)
+            for (int i = 0; i < ceil_div(N, small ? GEMM_SMALL_CELLS : GEMM_CELLS); ++i) t.push_back({0, i, r, 0});
         GemmTask* dt = (GemmTask*)al(t.size() * sizeof(GemmTask));
         RT_CHECK(hipMemcpy(dt, t.data(), t.size() * sizeof(GemmTask), hipMemcpyHostToDevice));
         PassDesc* dpd = (PassDesc*)al(sizeof(PassDesc));
@@ -1776,7 +1781,7 @@ void test_contraction(int which, int prec, int M, int K, int N, const double* A,
             RT_CHECK(hipMemcpy(dB, B, (size_t)K * N * 8, hipMemcpyHostToDevice));
             pd.Nd = M; pd.Nact = K; pd.Mact = dA; pd.qlout = dB; pd.phi_in = nullptr; pd.psi = dpsi;
             RT_CHECK(hipMemcpy(dpd, &pd, sizeof(pd), hipMemcpyHostToDevice));
-            launch_mgemm(prec, dpd, dt, (int)t.size(), nullptr);
+            launch_mgemm(prec, dpd, dt, (int)t.size(), nullptr, small);
             RT_CHECK(hipDeviceSynchronize());
             if (prec == P64) {
                 RT_CHECK(hipMemcpy(C, dpsi, (size_t)M * N * 8, hipMemcpyDeviceToHost));
@@ -1794,7 +1799,7 @@ void test_contraction(int which, int prec, int M, int K, int N, const double* A,
             }
             pd.Nd = K; pd.Nrows = M; pd.Drows = dA; pd.psi = dpsi; pd.out = dC; pd.zin = nullptr;
             RT_CHECK(hipMemcpy(dpd, &pd, sizeof(pd), hipMemcpyHostToDevice));
-            launch_dgemm(prec, dpd, dt, (int)t.size(), nullptr);
+            launch_dgemm(prec, dpd, dt, (int)t.size(), nullptr, small);
             RT_CHECK(hipDeviceSynchronize());
             RT_CHECK(hipMemcpy(C, dC, (size_t)M * N * 8, hipMemcpyDeviceToHost));
         }

@@ -178,6 +178,7 @@ private:
     PassDesc* d_pd = nullptr;
     GemmTask *d_mg = nullptr, *d_dgf = nullptr, *d_dga = nullptr;
     int n_mg = 0, n_dgf = 0, n_dga = 0;
+    bool sm_mg = false, sm_dgf = false, sm_dga = false;  // half-size work tiles (gemm_small)
     BndTask* d_bnd = nullptr;  // exit-face moment tasks of the D contraction's launch
     int n_bnd = 0;
     SweepTask* d_sw = nullptr;

@@ -348,8 +348,8 @@ __device__ __forceinline__ void contract_body(const PassDesc& d, const GemmTask 
     const double* __restrict__ phi_in = d.phi_in;
     const double* __restrict__ sigw = d.sigw;
     const bool hasq = qlout != nullptr, hasp = phi_in != nullptr;
-    const int c0 = tk.tile * GEMM_CELLS + wave * (CT * 16);
-    const int r0 = tk.rgroup * GEMM_ROWS;
+    const int c0 = tk.tile * (64 * CT) + wave * (CT * 16);
+    const int r0 = tk.rgroup * (16 * RT);
     const int kk = lane >> 4, li = lane & 15;
     int colc[CT], rowc[RT];
     bool colok[CT], rowok[RT];
@@ -467,7 +467,7 @@ __device__ __forceinline__ void contract_body(const PassDesc& d, const GemmTask 
 }
 
 template <typename T, int RT, int CT, bool MG, int NS, bool ADD = false, bool UL = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((sizeof(T) == 4 && !MG) ? 3 : 2))) void contract_kernel(const PassDesc* __restrict__ pds, const GemmTask* __restrict__ tasks) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 2 ? 4 : ((sizeof(T) == 4 && !MG) ? 3 : 2)))) void contract_kernel(const PassDesc* __restrict__ pds, const GemmTask* __restrict__ tasks) {
     __shared__ int rows_s[MG ? CONTRACT_KMAX : 1];
     const GemmTask tk = tasks[blockIdx.x];
     contract_body<T, RT, CT, MG, NS, ADD, UL>(pds[tk.prob], tk, rows_s);
@@ -483,7 +483,7 @@ __device__ inline void store_pd(PassDesc* dst) {
     for (int i = threadIdx.x; i < (int)(sizeof(PassDesc) / 8); i += blockDim.x) ((unsigned long long*)dst)[i] = src[i];
 }
 template <typename T, int RT, int CT, int NS, bool UL = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void contract_first_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 2 ? 4 : 2))) void contract_first_kernel(
     const PassDesc v, PassDesc* dst, const GemmTask* __restrict__ tasks) {
     __shared__ int rows_s[CONTRACT_KMAX];
     if (blockIdx.x == 0) store_pd(dst);
@@ -575,7 +575,7 @@ __device__ __forceinline__ void bnd_body(const PassDesc& d, const BndTask tk) {
             }
 }
 template <int RT, int CT, int NS, bool UL = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void contract_bnd_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 2 ? 4 : 2))) void contract_bnd_kernel(
     const PassDesc* __restrict__ pds, const GemmTask* __restrict__ tasks, int ntasks,
     const BndTask* __restrict__ btasks) {
     __shared__ int rows_s[1];
@@ -614,8 +614,8 @@ __global__ __launch_bounds__(256) void contract_bf16_kernel(const PassDesc* __re
     const double* __restrict__ phi_in = d.phi_in;
     const double* __restrict__ sigw = d.sigw;
     const bool hasq = qlout != nullptr, hasp = phi_in != nullptr;
-    const int c0 = tk.tile * GEMM_CELLS + wave * (CT * 16);
-    const int r0 = tk.rgroup * GEMM_ROWS;
+    const int c0 = tk.tile * (64 * CT) + wave * (CT * 16);
+    const int r0 = tk.rgroup * (16 * RT);
     const int kq = 4 * (lane >> 4), li = lane & 15;
     int colc[CT], rowc[RT];
     bool colok[CT], rowok[RT];
@@ -2882,19 +2882,33 @@ static void contract_first(int prec, const PassDesc& pd, PassDesc* d_pd, const G
     else launch_timed(contract_first_kernel<float, GEMM_RT, GEMM_CT, NS>, dim3(ntasks), dim3(256), 0, st, pd, d_pd, tasks);
 }
 
+// k steps in flight of the half-size tiles, whose stages hold half the registers
+constexpr int SMALL_NS_M = 4, SMALL_NS_D = 8;
+#define RT_SMALL GEMM_SMALL_RT, GEMM_SMALL_CT
+
 // Pipeline depth (k steps in flight) of the contractions: the default first, then the autotuner's
-// alternative (same accumulation order, so the same bits); BF16 operands keep their one shape.
-static void mgemm_any(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, const PassDesc* first) {
+// alternative (same accumulation order, so the same bits); BF16 operands and the half-size tiles
+// keep their one shape.
+static void mgemm_any(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, const PassDesc* first,
+                      bool small) {
     if (ntasks <= 0) return;
+    PassDesc* dst = const_cast<PassDesc*>(d_pd);
     if (prec == PBF16) {
-        launch_timed(contract_bf16_kernel<GEMM_RT, GEMM_CT, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        if (small) launch_timed(contract_bf16_kernel<RT_SMALL, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        else launch_timed(contract_bf16_kernel<GEMM_RT, GEMM_CT, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+    } else if (small) {
+        if (prec == PMIX) throw std::runtime_error("launch_mgemm: half-size tiles take one precision");
+        if (first && prec == P64) launch_timed(contract_first_kernel<double, RT_SMALL, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, *first, dst, tasks);
+        else if (first) launch_timed(contract_first_kernel<float, RT_SMALL, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, *first, dst, tasks);
+        else if (prec == P64) launch_timed(contract_kernel<double, RT_SMALL, true, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        else launch_timed(contract_kernel<float, RT_SMALL, true, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     } else {
         TuneTicket t;
         const int v = tune_choose({prec, 2, 0, 0, 0, ilog2(ntasks)}, 2, t);
         if (t.a) set_launch_events(t.a, t.b);
         if (first) {
-            if (v == 0) contract_first<2>(prec, *first, const_cast<PassDesc*>(d_pd), tasks, ntasks, st);
-            else contract_first<3>(prec, *first, const_cast<PassDesc*>(d_pd), tasks, ntasks, st);
+            if (v == 0) contract_first<2>(prec, *first, dst, tasks, ntasks, st);
+            else contract_first<3>(prec, *first, dst, tasks, ntasks, st);
         } else if (v == 0) contract_launch<true, 2>(prec, d_pd, tasks, ntasks, st);
         else contract_launch<true, 3>(prec, d_pd, tasks, ntasks, st);
         tune_commit(t);
@@ -2902,16 +2916,22 @@ static void mgemm_any(int prec, const PassDesc* d_pd, const GemmTask* tasks, int
     RT_HIP(hipGetLastError());
 }
 
-void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
-    mgemm_any(prec, d_pd, tasks, ntasks, st, nullptr);
+void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, bool small) {
+    mgemm_any(prec, d_pd, tasks, ntasks, st, nullptr, small);
 }
-void launch_mgemm_first(int prec, const PassDesc& pd, PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+void launch_mgemm_first(int prec, const PassDesc& pd, PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st,
+                        bool small) {
     if (prec != P64 && prec != P32) throw std::runtime_error("launch_mgemm_first: FP64 and FP32 passes only");
-    mgemm_any(prec, d_pd, tasks, ntasks, st, &pd);
+    mgemm_any(prec, d_pd, tasks, ntasks, st, &pd, small);
 }
 
-void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, bool small) {
     if (ntasks <= 0) return;
+    if (small) {
+        launch_timed(contract_kernel<double, RT_SMALL, false, SMALL_NS_D, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        RT_HIP(hipGetLastError());
+        return;
+    }
     TuneTicket t;
     const int v = tune_choose({P64, 4, 0, 0, 0, ilog2(ntasks)}, 2, t);
     if (t.a) set_launch_events(t.a, t.b);
@@ -2922,24 +2942,32 @@ void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, h
 }
 
 // The caller-layout forms take the default pipeline depths (this call times nothing).
-void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, const PassDesc* first) {
+void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, const PassDesc* first,
+                         bool small) {
     if (ntasks <= 0) return;
-    if (first)
-        launch_timed(contract_first_kernel<double, GEMM_RT, GEMM_CT, 2, true>, dim3(ntasks), dim3(256), 0, st, *first,
-                     const_cast<PassDesc*>(d_pd), tasks);
-    else
-        launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, true, 2, false, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+    PassDesc* dst = const_cast<PassDesc*>(d_pd);
+    if (first && small) launch_timed(contract_first_kernel<double, RT_SMALL, SMALL_NS_M, true>, dim3(ntasks), dim3(256), 0, st, *first, dst, tasks);
+    else if (first) launch_timed(contract_first_kernel<double, GEMM_RT, GEMM_CT, 2, true>, dim3(ntasks), dim3(256), 0, st, *first, dst, tasks);
+    else if (small) launch_timed(contract_kernel<double, RT_SMALL, true, SMALL_NS_M, false, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+    else launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, true, 2, false, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     RT_HIP(hipGetLastError());
 }
 void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt,
-                         hipStream_t st) {
+                         hipStream_t st, bool small) {
     if (ntasks <= 0) return;
-    launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 4, true>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
+    if (small) launch_timed(contract_bnd_kernel<RT_SMALL, SMALL_NS_D, true>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
+    else launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 4, true>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
     RT_HIP(hipGetLastError());
 }
 
-void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt, hipStream_t st) {
+void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt, hipStream_t st,
+                      bool small) {
     if (ntasks <= 0) return;
+    if (small) {
+        launch_timed(contract_bnd_kernel<RT_SMALL, SMALL_NS_D>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
+        RT_HIP(hipGetLastError());
+        return;
+    }
     TuneTicket t;
     const int v = tune_choose({P64, 3, 0, 0, 1, ilog2(ntasks)}, 2, t);
     if (t.a) set_launch_events(t.a, t.b);
@@ -2949,10 +2977,15 @@ void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, c
     RT_HIP(hipGetLastError());
 }
 
-void launch_dgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st) {
+void launch_dgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, bool small) {
     if (ntasks <= 0) return;
     if (prec == PBF16) {
-        launch_timed(contract_bf16_kernel<GEMM_RT, GEMM_CT, false>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        if (small) launch_timed(contract_bf16_kernel<RT_SMALL, false>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        else launch_timed(contract_bf16_kernel<GEMM_RT, GEMM_CT, false>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+    } else if (small) {
+        if (prec == PMIX) throw std::runtime_error("launch_dgemm: half-size tiles take one precision");
+        if (prec == P64) launch_timed(contract_kernel<double, RT_SMALL, false, SMALL_NS_D>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        else launch_timed(contract_kernel<float, RT_SMALL, false, SMALL_NS_D>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     } else {
         TuneTicket t;
         const int v = tune_choose({prec, 3, 0, 0, 0, ilog2(ntasks)}, 2, t);

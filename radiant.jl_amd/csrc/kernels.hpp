@@ -136,8 +136,9 @@ size_t sweep_lds_bytes(int prec, int Nx, int Ny, int Nz, int Nmat, int nbuf);
 
 // _first: the launch takes the PassDesc by value and stores it in d_pd for the launches that follow it
 // on the stream (single problems, FP64 and FP32).
-void launch_mgemm_first(int prec, const PassDesc& pd, PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
-void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
+void launch_mgemm_first(int prec, const PassDesc& pd, PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st,
+                        bool small);
+void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, bool small = false);
 // The same for the kernels that come before the contraction.
 void launch_bndin_first(const PassDesc& pd, PassDesc* d_pd, int total, hipStream_t st);
 void launch_fp_source_first(const PassDesc& pd, PassDesc* d_pd, long n, hipStream_t st);
@@ -147,14 +148,14 @@ struct BndTask { int code, rgroup, tile, pad; };  // code: 2 * axis + face
 constexpr int BND_ROWS = 32;    // half-range moments per boundary task
 constexpr int BND_CELLS = 128;  // face positions (times face moments) per boundary task
 void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt,
-                      hipStream_t st);
+                      hipStream_t st, bool small);
 // The FP64 contractions of one problem on states in the caller's layout (PassDesc::ul_np)
 void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st,
-                         const PassDesc* first);
+                         const PassDesc* first, bool small);
 void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt,
-                         hipStream_t st);
+                         hipStream_t st, bool small);
 // FP64 D contraction of (psi + psi_add), one problem (PassDesc::psi_add non-null)
-void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
+void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, bool small);
 void launch_sweep(int prec, const PassDesc* d_pd, const SweepTask* tasks, int ntasks, int ppt, int nbuf,
                   int block, size_t lds, hipStream_t st);
 // 1D/2D wave-per-direction sweep (rows per lane 1, 2 or 4; -1 when the grid does not fit).
@@ -228,7 +229,7 @@ void launch_bfp_out(const PassDesc* d_pd, long n, hipStream_t st);
 void take_launch_events(hipEvent_t* start, hipEvent_t* stop);
 void launch_sweep_3d_ho(int prec, const PassDesc* d_pd, int Nd, int Kx, int Ky, int Kz, bool fc, size_t lds,
                         hipStream_t st);
-void launch_dgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st);
+void launch_dgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, bool small = false);
 void launch_bndmom(const PassDesc* d_pd, int nprob, int max_items, hipStream_t st);
 
 // Order of the work tiles of one contraction: task i -> (cell tile, row group).  The row groups of
@@ -254,6 +255,17 @@ constexpr int GEMM_RT = 4;                      // 16-row MFMA tiles per wave
 constexpr int GEMM_CT = 4;                      // 16-cell MFMA tiles per wave
 constexpr int GEMM_ROWS = 16 * GEMM_RT;         // rows per work tile
 constexpr int GEMM_CELLS = 4 * 16 * GEMM_CT;    // cells per work tile (4 waves)
+// Problems whose work tiles of that size would fill less than one round of two workgroups per CU
+// take tiles of half the rows and half the cells (the sums keep their order, so the same bits):
+// four times the waves in flight, each with its operands reused half as often, which the L2 covers.
+// D of 128 moments, 128 directions, 16384 cells in FP64 30 -> 24 us, of 36 moments 23 -> 12 us; FP32 M and
+// D of a 128 x 128 plane 12 and 18 -> 11 and 11 us, of a 24 x 26 x 21 box 11 and 11 -> 7 and 6 us.
+constexpr int GEMM_SMALL_RT = 2, GEMM_SMALL_CT = 2;
+constexpr int GEMM_SMALL_ROWS = 16 * GEMM_SMALL_RT, GEMM_SMALL_CELLS = 4 * 16 * GEMM_SMALL_CT;
+constexpr int GEMM_FILL = 512;
+inline bool gemm_small(int rows, int Nc) {
+    return (long)((rows + GEMM_ROWS - 1) / GEMM_ROWS) * ((Nc + GEMM_CELLS - 1) / GEMM_CELLS) < GEMM_FILL;
+}
 constexpr int CONTRACT_KMAX = 1024;             // active moments at most (row map held in LDS)
 
 // Out-of-group + volume source of group g (sn_flux.jl:175-179):
