@@ -10,6 +10,7 @@
 #include "sweep_hog.hpp"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -592,14 +593,8 @@ Problem::Problem(const rt_problem_desc& d, hipStream_t stream) {
         d_dgf = gemm_tasks(Np, n_dgf, sm_dgf);
         d_dga = gemm_tasks(Nact, n_dga, sm_dga);
         if (state_mode == RT_STATE_FAITHFUL || has_bc) {
-            std::vector<BndTask> t;
-            for (int ax = 0; ax < ndims; ++ax)
-                for (int f = 0; f < 2; ++f)
-                    for (int i = 0; i < ceil_div((int)npos[ax], BND_CELLS); ++i)
-                        for (int r = 0; r < ceil_div(Nps, BND_ROWS); ++r) t.push_back({2 * ax + f, r, i, 0});
-            n_bnd = (int)t.size();
-            d_bnd = dalloc<BndTask>(std::max<size_t>(1, t.size()));
-            if (n_bnd) upload(d_bnd, t, st);
+            bnd.rg = ceil_div(Nps, BND_ROWS);
+            for (int ax = 0; ax < ndims; ++ax) bnd.cells[ax] = ceil_div((int)npos[ax], BND_CELLS);
         }
         std::vector<SweepTask> sw(Nd);
         for (int n = 0; n < Nd; ++n) sw[n] = {0, n};
@@ -648,10 +643,13 @@ Problem::Problem(const rt_problem_desc& d, hipStream_t stream) {
         // ---- reductions
         rw.partial = dalloc<double>(RED_BLOCKS);
         rw.scal = dalloc<double>(128);
-        // pinned: 128 scalar slots, then the two Gram-Schmidt items of a classical Arnoldi step
-        RT_CHECK(hipHostMalloc((void**)&h_scal, 128 * sizeof(double) + 2 * sizeof(GsItem), hipHostMallocDefault));
-        d_gsi = dalloc<GsItem>(2);
-        d_gspart = dalloc<double>((size_t)GS_BPI_MAX * GS_KMAX);
+        // pinned: 128 scalar slots, then the counter the host polls
+        RT_CHECK(hipHostMalloc((void**)&h_scal, (KRY_FLAG + 1) * sizeof(double), hipHostMallocDefault));
+        std::memset(h_scal, 0, (KRY_FLAG + 1) * sizeof(double));
+        aw.part = dalloc<double>((size_t)ARN_BLOCKS * (2 * GS_KMAX + 1) + (size_t)GS_KMAX * (GS_KMAX + 1));
+        aw.L = aw.part + (size_t)ARN_BLOCKS * (2 * GS_KMAX + 1);
+        aw.h = aw.L + (size_t)GS_KMAX * GS_KMAX;
+        RT_CHECK(hipHostGetDevicePointer((void**)&aw.host, h_scal, 0));
         d_Vptr = dalloc<double*>(64);
         d_y = dalloc<double>(64);
         RT_CHECK(hipStreamSynchronize(st));
@@ -728,6 +726,20 @@ double* Problem::vec(const std::string& name, size_t n) {
     void* p = dev_alloc(n * sizeof(double));
     pool[key] = (double*)p;
     return (double*)p;
+}
+
+// Waits until the kernel that sends seq to the pinned counter has done so: polls (a synchronising
+// call returns some 10 us after the kernel's end), and after a while leaves the wait to the stream.
+void Problem::wait_host(unsigned long long seq) {
+    const volatile unsigned long long* flag = (const volatile unsigned long long*)(h_scal + KRY_FLAG);
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int i = 0;; ++i) {
+        if (__atomic_load_n((const unsigned long long*)flag, __ATOMIC_ACQUIRE) == seq) return;
+        if ((i & 255) == 255 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+    }
+    RT_CHECK(hipStreamSynchronize(st));
+    if (__atomic_load_n((const unsigned long long*)flag, __ATOMIC_ACQUIRE) != seq)
+        throw Error(RT_EDEVICE, "the device did not report its results");
 }
 
 double Problem::dot(const double* a, const double* b, size_t n) {
@@ -883,8 +895,8 @@ void Problem::launch_pass(PassDesc& pd, int prec, bool full_rows) {
         const GemmTask* dg = full_rows ? d_dgf : d_dga;
         const int n_dg = full_rows ? n_dgf : n_dga;
         const bool sm = full_rows ? sm_dgf : sm_dga;
-        if (caller) launch_dgemm_caller(d_pd, dg, n_dg, d_bnd, merged ? n_bnd : 0, st, sm);
-        else if (merged) launch_dgemm_bnd(d_pd, dg, n_dg, d_bnd, n_bnd, st, sm);
+        if (caller) launch_dgemm_caller(d_pd, dg, n_dg, merged ? bnd : BndTiles{}, st, sm);
+        else if (merged) launch_dgemm_bnd(d_pd, dg, n_dg, bnd, st, sm);
         else launch_dgemm(prec, d_pd, dg, n_dg, st, sm);
     });
     if (pd.bout_x && !merged) timed(3, [&] { launch_bndmom(d_pd, 1, (int)nb, st); });
@@ -1070,11 +1082,10 @@ static double rho_estimate(double r0, double r, int64_t it) {  // krylov_state.j
 }
 
 // tools/gmres.jl:35-133 -- restarted GMRES(m), modified Gram-Schmidt, Givens rotations.
-// The MGS chain runs on the device (each kernel reads its coefficient from a scalar slot and
-// reduces the next dot product); the host reads one H column per Arnoldi step.  Two options
+// The host reads one H column per Arnoldi step (launch_arnoldi).  Two options
 // serve the inner solves of the mixed-precision refinement, which need no parity with
 // gmres.jl's iteration counts: zero_guess (z = 0, so the first residual is c without a pass) and
-// cgs (classical Gram-Schmidt in two passes over the basis instead of the MGS chain).
+// cgs (classical instead of modified Gram-Schmidt).
 template <class MV>
 void Problem::gmres(size_t n, double* z, MV matvec, const double* c, int m, int64_t maxit_, double tol_,
                     int64_t& iter, double& resid, bool& conv, double& rho, const std::string& tag, bool zero_guess,
@@ -1092,6 +1103,8 @@ void Problem::gmres(size_t n, double* z, MV matvec, const double* c, int m, int6
     double* w = vec(tag + "w", n);
     double* r = vec(tag + "r", n);
     RT_CHECK(hipMemcpyAsync(d_Vptr, V.data(), (m + 1) * sizeof(double*), hipMemcpyHostToDevice, st));
+    BasisTab tab{};
+    for (int i = 0; i < std::min(m + 1, GS_KMAX); ++i) tab.p[i] = V[i];
     std::vector<double> H((size_t)(m + 1) * m, 0.0), cs(m, 0.0), sn(m, 0.0), gv(m + 1, 0.0);
     auto h = [&](int i, int j) -> double& { return H[i + (size_t)(m + 1) * j]; };
     iter = 0; resid = 1.0; conv = false;
@@ -1118,23 +1131,16 @@ void Problem::gmres(size_t n, double* z, MV matvec, const double* c, int m, int6
         for (int j = 0; j < m; ++j) {
             if (iter >= maxit_) break;
             matvec(w, V[j]); ++iter;
-            if (cgs) {
-                // classical Gram-Schmidt in two passes over the basis: h = V^T w, then
-                // w -= V h with |w|^2 (the item is reused after the step's synchronisation)
-                GsItem* h_gsi = (GsItem*)(h_scal + 128);
-                const int bpi = gs_blocks((long)n);
-                h_gsi[0] = GsItem{(const double* const*)d_Vptr, nullptr, w, rw.scal, (long)n, j + 1, bpi};
-                h_gsi[1] = GsItem{(const double* const*)d_Vptr, rw.scal, w, rw.scal + j + 1, (long)n, j + 1, bpi};
-                RT_CHECK(hipMemcpyAsync(d_gsi, h_gsi, 2 * sizeof(GsItem), hipMemcpyHostToDevice, st));
-                launch_gs(d_gsi, 1, j + 1, bpi, false, false, d_gspart, st);
-                launch_gs(d_gsi + 1, 1, j + 1, bpi, true, true, d_gspart, st);
-            } else {
+            if (m <= GS_KMAX || cgs) {
+                launch_arnoldi(tab, w, V[j + 1], (long)n, j + 1, !cgs, aw, ++seq, st);
+                wait_host(seq);
+            } else {  // bases beyond the kernels' size: the chain of reductions, vector by vector
                 k_dot(rw, 0, w, V[0], n, st);
                 for (int i = 0; i <= j; ++i) k_mgs(rw, i, i + 1, w, V[i], i < j ? V[i + 1] : nullptr, n, st);
+                k_scale_by_inv_slot(V[j + 1], w, rw.scal, j + 1, n, st);
+                RT_CHECK(hipMemcpyAsync(h_scal, rw.scal, (j + 2) * sizeof(double), hipMemcpyDeviceToHost, st));
+                RT_CHECK(hipStreamSynchronize(st));
             }
-            k_scale_by_inv_slot(V[j + 1], w, rw.scal, j + 1, n, st);
-            RT_CHECK(hipMemcpyAsync(h_scal, rw.scal, (j + 2) * sizeof(double), hipMemcpyDeviceToHost, st));
-            RT_CHECK(hipStreamSynchronize(st));
             for (int i = 0; i <= j; ++i) h(i, j) = h_scal[i];
             const double hjp1 = std::sqrt(h_scal[j + 1]);
             h(j + 1, j) = hjp1;

@@ -179,8 +179,7 @@ private:
     GemmTask *d_mg = nullptr, *d_dgf = nullptr, *d_dga = nullptr;
     int n_mg = 0, n_dgf = 0, n_dga = 0;
     bool sm_mg = false, sm_dgf = false, sm_dga = false;  // half-size work tiles (gemm_small)
-    BndTask* d_bnd = nullptr;  // exit-face moment tasks of the D contraction's launch
-    int n_bnd = 0;
+    BndTiles bnd;  // exit-face moment tiles of the D contraction's launch
     SweepTask* d_sw = nullptr;
     int sw_ppt = 1, sw_block = 64, sw_nbuf[3] = {2, 2, 2};
     int rows_per_lane = -1;   // > 0: 1D/2D wave-per-direction sweep
@@ -195,8 +194,9 @@ private:
     double* vec(const std::string& name, size_t n);
     RedWork rw{};
     double* h_scal = nullptr;   // pinned mirror of the scalar slots
-    GsItem* d_gsi = nullptr;    // the two Gram-Schmidt items of a classical Arnoldi step
-    double* d_gspart = nullptr; // their block partials
+    ArnoldiWork aw{};           // workspace of the Arnoldi steps
+    unsigned long long seq = 0; // results asked of the device so far (the pinned counter's next value)
+    void wait_host(unsigned long long seq);
     double** d_Vptr = nullptr;  // device table of Krylov basis pointers
     double* d_y = nullptr;
 

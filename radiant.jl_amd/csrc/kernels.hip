@@ -496,9 +496,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 2 ? 4
 // nor writes to.  One thread per moment and position, in a launch of its own, took 10 us (2D, 128 x 128,
 // 128 directions) and 22 us (3D, 40 x 37 x 42, 80 directions); with the PassDesc launch gone too a
 // pass of the first went from 115 to 101 us, of a 31 x 29 x 30 box from 130 to 113 us.
-__device__ __forceinline__ void bnd_body(const PassDesc& d, const BndTask tk) {
+__device__ __forceinline__ void bnd_body(const PassDesc& d, const BndTiles bt, int b) {
     constexpr int RT = 2, CT = 2, NS = 4;
-    const int ax = tk.code >> 1, f = tk.code & 1;
+    int ax = 0;  // tile b: axis, face, cell tile, row group
+    while (ax < 2 && b >= 2 * bt.rg * bt.cells[ax]) b -= 2 * bt.rg * bt.cells[ax++];
+    const int f = b / (bt.rg * bt.cells[ax]), rest = b - f * bt.rg * bt.cells[ax];
+    const int tile = rest / bt.rg, rgroup = rest - tile * bt.rg;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kk = lane >> 4, li = lane & 15;
     const int fm_ = ax == 0 ? d.fm_x : (ax == 1 ? d.fm_y : d.fm_z), fm = fm_ > 1 ? fm_ : 1;
     const int N = (ax == 0 ? d.Ny * d.Nz : (ax == 1 ? d.Nx * d.Nz : d.Nx * d.Ny)) * fm;
@@ -508,7 +511,7 @@ __device__ __forceinline__ void bnd_body(const PassDesc& d, const BndTask tk) {
     const int* __restrict__ lst = (ax == 0 ? d.exlist_x : (ax == 1 ? d.exlist_y : d.exlist_z)) + f * d.Nd;
     double* out = ax == 0 ? d.bout_x : (ax == 1 ? d.bout_y : d.bout_z);
     const double* zin = ax == 0 ? d.bzin_x : (ax == 1 ? d.bzin_y : d.bzin_z);
-    const int c0 = tk.tile * BND_CELLS + wave * (CT * 16), r0 = tk.rgroup * BND_ROWS;
+    const int c0 = tile * BND_CELLS + wave * (CT * 16), r0 = rgroup * BND_ROWS;
     int colc[CT], rowc[RT];
 #pragma unroll
     for (int u = 0; u < CT; ++u) colc[u] = c0 + 16 * u + li < N ? c0 + 16 * u + li : N - 1;
@@ -577,10 +580,10 @@ __device__ __forceinline__ void bnd_body(const PassDesc& d, const BndTask tk) {
 template <int RT, int CT, int NS, bool UL = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 2 ? 4 : 2))) void contract_bnd_kernel(
     const PassDesc* __restrict__ pds, const GemmTask* __restrict__ tasks, int ntasks,
-    const BndTask* __restrict__ btasks) {
+    const BndTiles bt) {
     __shared__ int rows_s[1];
     if ((int)blockIdx.x < ntasks) contract_body<double, RT, CT, false, NS, false, UL>(pds[0], tasks[blockIdx.x], rows_s);
-    else bnd_body(pds[0], btasks[blockIdx.x - ntasks]);
+    else bnd_body(pds[0], bt, (int)blockIdx.x - ntasks);
 }
 
 // FP64 and FP32 passes of different problems in one launch (PassDesc::prec per workgroup).
@@ -2952,27 +2955,28 @@ void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks
     else launch_timed(contract_kernel<double, GEMM_RT, GEMM_CT, true, 2, false, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     RT_HIP(hipGetLastError());
 }
-void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt,
-                         hipStream_t st, bool small) {
+void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTiles& bt, hipStream_t st,
+                         bool small) {
     if (ntasks <= 0) return;
-    if (small) launch_timed(contract_bnd_kernel<RT_SMALL, SMALL_NS_D, true>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
-    else launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 4, true>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
+    const int nbt = bnd_count(bt);
+    if (small) launch_timed(contract_bnd_kernel<RT_SMALL, SMALL_NS_D, true>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, bt);
+    else launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 4, true>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, bt);
     RT_HIP(hipGetLastError());
 }
 
-void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt, hipStream_t st,
-                      bool small) {
+void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTiles& bt, hipStream_t st, bool small) {
     if (ntasks <= 0) return;
+    const int nbt = bnd_count(bt);
     if (small) {
-        launch_timed(contract_bnd_kernel<RT_SMALL, SMALL_NS_D>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
+        launch_timed(contract_bnd_kernel<RT_SMALL, SMALL_NS_D>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, bt);
         RT_HIP(hipGetLastError());
         return;
     }
     TuneTicket t;
     const int v = tune_choose({P64, 3, 0, 0, 1, ilog2(ntasks)}, 2, t);
     if (t.a) set_launch_events(t.a, t.b);
-    if (v == 0) launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 4>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
-    else launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 2>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, btasks);
+    if (v == 0) launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 4>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, bt);
+    else launch_timed(contract_bnd_kernel<GEMM_RT, GEMM_CT, 2>, dim3(ntasks + nbt), dim3(256), 0, st, d_pd, tasks, ntasks, bt);
     tune_commit(t);
     RT_HIP(hipGetLastError());
 }

@@ -142,18 +142,18 @@ void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int nta
 // The same for the kernels that come before the contraction.
 void launch_bndin_first(const PassDesc& pd, PassDesc* d_pd, int total, hipStream_t st);
 void launch_fp_source_first(const PassDesc& pd, PassDesc* d_pd, long n, hipStream_t st);
-// FP64 D contraction of one problem with the half-range moments of its exit faces (nbt boundary
-// tasks, as a pass with PassDesc::bout_* wants them) in one launch.
-struct BndTask { int code, rgroup, tile, pad; };  // code: 2 * axis + face
-constexpr int BND_ROWS = 32;    // half-range moments per boundary task
-constexpr int BND_CELLS = 128;  // face positions (times face moments) per boundary task
-void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt,
-                      hipStream_t st, bool small);
+// FP64 D contraction of one problem with the half-range moments of its exit faces (as a pass with
+// PassDesc::bout_* wants them) in one launch: the boundary work tiles follow the contraction's.
+constexpr int BND_ROWS = 32;    // half-range moments per boundary tile
+constexpr int BND_CELLS = 128;  // face positions (times face moments) per boundary tile
+struct BndTiles { int rg = 0, cells[3] = {0, 0, 0}; };  // row groups, and cell tiles of a face per axis
+inline int bnd_count(const BndTiles& b) { return 2 * b.rg * (b.cells[0] + b.cells[1] + b.cells[2]); }
+void launch_dgemm_bnd(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTiles& bt, hipStream_t st, bool small);
 // The FP64 contractions of one problem on states in the caller's layout (PassDesc::ul_np)
 void launch_mgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st,
                          const PassDesc* first, bool small);
-void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTask* btasks, int nbt,
-                         hipStream_t st, bool small);
+void launch_dgemm_caller(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, const BndTiles& bt, hipStream_t st,
+                         bool small);
 // FP64 D contraction of (psi + psi_add), one problem (PassDesc::psi_add non-null)
 void launch_dgemm_add(const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, bool small);
 void launch_sweep(int prec, const PassDesc* d_pd, const SweepTask* tasks, int ntasks, int ppt, int nbuf,
@@ -335,6 +335,23 @@ int gs_blocks(long n);   // the block count of an item of length n
 void launch_gs(const GsItem* items, int nitems, int kmax, int bpi_max, bool update, bool norm, double* partial,
                hipStream_t st);
 void launch_vecops(const VecItem* items, int nitems, int blocks_per_item, hipStream_t st);
+
+// Arnoldi step of a single problem (krylov.hip): orthogonalises w against the k vectors of the basis
+// (modified Gram-Schmidt in its triangular-solve form, or classical), writes vnext = w / |w| when
+// |w| > 0, and sends the column h_0..h_(k-1), |w|^2 to host[0..k], then seq to host[KRY_FLAG].  The
+// modified form keeps the basis' inner products in L, so a cycle starts at k = 1 and goes on by one.
+constexpr int ARN_BLOCKS = 1024;          // blocks of a reduction at most
+constexpr long ARN_SMALL_READS = 1 << 16;  // n * k of the one-workgroup form at most
+constexpr int KRY_FLAG = 128;             // index of the counter in the pinned results
+struct BasisTab { const double* p[GS_KMAX]; };
+struct ArnoldiWork {
+    double* part;  // ARN_BLOCKS * (2 * GS_KMAX + 1) partial sums
+    double* L;     // GS_KMAX * GS_KMAX
+    double* h;     // GS_KMAX
+    double* host;  // pinned: KRY_FLAG results and the counter
+};
+void launch_arnoldi(const BasisTab& V, double* w, double* vnext, long n, int k, bool mgs, const ArnoldiWork& aw,
+                    unsigned long long seq, hipStream_t st);
 
 // Layout converters of the host boundary (Radiant order <-> device order).
 void k_phi_to_radiant(double* dst, const double* phi_all, int G, int Np, int Nc, int c0, int nc, hipStream_t st);

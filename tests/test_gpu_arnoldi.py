@@ -1,0 +1,20 @@
+"""Arnoldi steps of the FP64 solve at the sizes where their form changes: state lengths around the
+one-workgroup limit (16 moments x N cells + 32 boundary moments: 8176, 8192, 8208), tiny ones, long
+ones, and restarts around the 33 vectors the kernels hold (34: the chain of reductions).  The
+iteration counts and the flux are the oracle's (both converge to 1e-12; they differ by rounding)."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("cells,restart", [(2, 30), (509, 30), (510, 30), (510, 3), (511, 30), (511, 12), (63, 33), (63, 34)])
+def test_solve_forms(oracle, cells, restart):
+    from radiant_hip import problems, solver
+    from util import rel_err
+    p = problems.small_problem(1, N=cells, G=2, L=3, quad_order=16, seed=31, tol=1e-12, bc=[1, 0])
+    p.restart = restart
+    ref, rst = oracle.solve(p)
+    phi, st = solver.compute_flux(p)
+    print(cells, restart, rel_err(phi, ref), [s["niter"] for s in st], [s["niter"] for s in rst], flush=True)
+    assert rel_err(phi, ref) < 1e-10 and all(s["converged"] for s in st)
+    assert [s["niter"] for s in st] == [s["niter"] for s in rst]
