@@ -651,7 +651,6 @@ Problem::Problem(const rt_problem_desc& d, hipStream_t stream) {
         aw.h = aw.L + (size_t)GS_KMAX * GS_KMAX;
         RT_CHECK(hipHostGetDevicePointer((void**)&aw.host, h_scal, 0));
         d_Vptr = dalloc<double*>(64);
-        d_y = dalloc<double>(64);
         RT_CHECK(hipStreamSynchronize(st));
     } catch (...) {
         (void)hipStreamSynchronize(st);
@@ -743,10 +742,18 @@ void Problem::wait_host(unsigned long long seq) {
 }
 
 double Problem::dot(const double* a, const double* b, size_t n) {
-    k_dot(rw, 0, a, b, n, st);
-    RT_CHECK(hipMemcpyAsync(h_scal, rw.scal, sizeof(double), hipMemcpyDeviceToHost, st));
-    RT_CHECK(hipStreamSynchronize(st));
+    const DotTab t{{a}, {b}, 1};
+    launch_dots(t, (long)n, aw, ++seq, st);
+    wait_host(seq);
     return h_scal[0];
+}
+
+void Problem::dot2(const double* a, const double* b, const double* c, const double* d, size_t n, double& ab, double& cd) {
+    const DotTab t{{a, c}, {b, d}, 2};
+    launch_dots(t, (long)n, aw, ++seq, st);
+    wait_host(seq);
+    ab = h_scal[0];
+    cd = h_scal[1];
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1083,8 +1090,7 @@ static double rho_estimate(double r0, double r, int64_t it) {  // krylov_state.j
 
 // tools/gmres.jl:35-133 -- restarted GMRES(m), modified Gram-Schmidt, Givens rotations.
 // The host reads one H column per Arnoldi step (launch_arnoldi).  Two options
-// serve the inner solves of the mixed-precision refinement, which need no parity with
-// gmres.jl's iteration counts: zero_guess (z = 0, so the first residual is c without a pass) and
+// serve: zero_guess (z stands for zero and need not be set; the first residual is c without a pass) and
 // cgs (classical instead of modified Gram-Schmidt).
 template <class MV>
 void Problem::gmres(size_t n, double* z, MV matvec, const double* c, int m, int64_t maxit_, double tol_,
@@ -1102,7 +1108,6 @@ void Problem::gmres(size_t n, double* z, MV matvec, const double* c, int m, int6
     for (int i = 0; i <= m; ++i) V[i] = vec(tag + "V" + std::to_string(i), n);
     double* w = vec(tag + "w", n);
     double* r = vec(tag + "r", n);
-    RT_CHECK(hipMemcpyAsync(d_Vptr, V.data(), (m + 1) * sizeof(double*), hipMemcpyHostToDevice, st));
     BasisTab tab{};
     for (int i = 0; i < std::min(m + 1, GS_KMAX); ++i) tab.p[i] = V[i];
     std::vector<double> H((size_t)(m + 1) * m, 0.0), cs(m, 0.0), sn(m, 0.0), gv(m + 1, 0.0);
@@ -1110,21 +1115,24 @@ void Problem::gmres(size_t n, double* z, MV matvec, const double* c, int m, int6
     iter = 0; resid = 1.0; conv = false;
     double resid0 = std::numeric_limits<double>::quiet_NaN();
     bool first = true;
+    bool empty = zero_guess;  // z stands for zero and has not been written
     while (iter < maxit_ && !conv) {
-        const bool skip = first && zero_guess;  // z = 0: the initial residual is c, no pass needed
+        // z = 0: the initial residual is c, no pass needed (gmres.jl counts one all the same)
+        const bool skip = first && zero_guess;
         first = false;
+        double beta = bnorm;
         if (skip) {
-            k_copy(r, c, n, st);
+            if (!cgs) ++iter;
         } else {
-            matvec(r, z); ++iter;
-            k_neg_add(r, c, n, st);  // r = c - r  (state_scale!(-1) ; state_axpy!(1, c))
+            matvec(w, z); ++iter;
+            launch_residual(r, c, w, (long)n, aw, ++seq, st);  // r = c - (I - A) z
+            wait_host(seq);
+            beta = std::sqrt(h_scal[0]);
         }
-        const double beta = skip ? bnorm : norm(r, n);
         resid = beta / bnorm;
         if (std::isnan(resid0)) resid0 = resid;
         if (resid < tol_) { conv = true; break; }
-        k_copy(V[0], r, n, st);
-        k_scale(V[0], 1.0 / beta, n, st);
+        launch_scale_copy(V[0], skip ? c : r, 1.0 / beta, (long)n, st);
         std::fill(gv.begin(), gv.end(), 0.0);
         gv[0] = beta;
         int k = 0;
@@ -1170,12 +1178,14 @@ void Problem::gmres(size_t n, double* z, MV matvec, const double* c, int m, int6
         for (int i0 = 0; i0 < k; i0 += 32) {
             const int kk = std::min(32, k - i0);
             Vals32 v{};
-            for (int t = 0; t < kk; ++t) v.v[t] = y[i0 + t];
-            k_set_vals(v, d_y, kk, st);
-            k_lincomb(z, (const double* const*)(d_Vptr + i0), d_y, kk, n, st);
+            BasisTab tb{};
+            for (int t = 0; t < kk; ++t) { v.v[t] = y[i0 + t]; tb.p[t] = V[i0 + t]; }
+            launch_combine(z, tb, v, kk, !empty, (long)n, st);
+            empty = false;
         }
         if (conv) break;
     }
+    if (empty) k_fill(z, 0.0, n, st);
     rho = rho_estimate(resid0, resid, iter);
 }
 
@@ -1188,37 +1198,70 @@ void Problem::anderson(size_t n, double* z, FP fixedpoint, int64_t& iter, double
     double* fo = vec("afo", n);
     double* go = vec("ago", n);
     std::vector<double*> dF, dG;
+    std::vector<double> Nm, Gm;  // inner products of the differences: with the Tikhonov term, kept
+    const bool fused = m <= AND_DEPTH;
+    AndersonTab t{};
     iter = 0; resid = 1.0; conv = false;
     double resid0 = std::numeric_limits<double>::quiet_NaN();
     for (int64_t it = 1; it <= maxit; ++it) {
         fixedpoint(g, z); ++iter;
-        k_copy(f, g, n, st);
-        k_axpy(-1.0, z, f, n, st);
-        const double fnorm = norm(f, n);
-        const double sc = std::max(std::max(norm(z, n), norm(g, n)), 1e-16);
+        // history of depth m (push!, then popfirst! when longer than m): reuse the oldest buffers
+        const int old = (int)dF.size();
+        if (it > 1) {
+            double *a, *b;
+            if (old < m) {
+                a = vec("adF" + std::to_string(old), n);
+                b = vec("adG" + std::to_string(old), n);
+            } else {
+                a = dF.front(); b = dG.front();
+                dF.erase(dF.begin()); dG.erase(dG.begin());
+            }
+            dF.push_back(a); dG.push_back(b);
+        }
+        const int mk = (int)dF.size();
+        double fnorm, sc;
+        std::vector<double> bb(mk);
+        if (fused) {
+            // one pass forms f, the differences and every inner product; the entries of the older
+            // differences are those of the iterations that formed them (shifted when the oldest goes)
+            t.g = g; t.z = z; t.f = f; t.fo = fo; t.go = go; t.mk = mk;
+            for (int i = 0; i < mk; ++i) { t.dF[i] = dF[i]; t.dG[i] = dG[i]; }
+            launch_anderson(t, (long)n, aw, ++seq, st);
+            wait_host(seq);
+            fnorm = std::sqrt(h_scal[0]);
+            sc = std::max(std::max(std::sqrt(h_scal[1]), std::sqrt(h_scal[2])), 1e-16);
+            if (mk > 0) {
+                std::vector<double> G2((size_t)mk * mk, 0.0);
+                const int sh = old == mk ? 1 : 0;  // the oldest left
+                for (int i = 0; i + 1 < mk; ++i)
+                    for (int j = 0; j + 1 < mk; ++j) G2[i + (size_t)mk * j] = Gm[(i + sh) + (size_t)old * (j + sh)];
+                for (int i = 0; i < mk; ++i) {
+                    bb[i] = h_scal[3 + i];
+                    G2[i + (size_t)mk * (mk - 1)] = G2[(mk - 1) + (size_t)mk * i] = h_scal[3 + AND_DEPTH + i];
+                }
+                Gm.swap(G2);
+                Nm = Gm;
+            }
+        } else {
+            k_copy(f, g, n, st);
+            k_axpy(-1.0, z, f, n, st);
+            fnorm = norm(f, n);
+            sc = std::max(std::max(norm(z, n), norm(g, n)), 1e-16);
+        }
         resid = fnorm / sc;
         if (std::isnan(resid0)) resid0 = resid;
         if (resid < tol) { conv = true; break; }
         if (it == 1) {
             k_axpy(1.0, f, z, n, st);
         } else {
-            // history of depth m (push!, then popfirst! when longer than m): reuse the oldest buffers
-            double *a, *b;
-            if ((int)dF.size() < m) {
-                a = vec("adF" + std::to_string(dF.size()), n);
-                b = vec("adG" + std::to_string(dG.size()), n);
-            } else {
-                a = dF.front(); b = dG.front();
-                dF.erase(dF.begin()); dG.erase(dG.begin());
-            }
-            dF.push_back(a); dG.push_back(b);
-            k_copy(a, f, n, st); k_axpy(-1.0, fo, a, n, st);
-            k_copy(b, g, n, st); k_axpy(-1.0, go, b, n, st);
-            const int mk = (int)dF.size();
-            std::vector<double> Nm((size_t)mk * mk), bb(mk);
-            for (int i = 0; i < mk; ++i) {
-                bb[i] = dot(dF[i], f, n);
-                for (int j = 0; j < mk; ++j) Nm[i + (size_t)mk * j] = dot(dF[i], dF[j], n);
+            if (!fused) {
+                k_copy(dF.back(), f, n, st); k_axpy(-1.0, fo, dF.back(), n, st);
+                k_copy(dG.back(), g, n, st); k_axpy(-1.0, go, dG.back(), n, st);
+                Nm.assign((size_t)mk * mk, 0.0);
+                for (int i = 0; i < mk; ++i) {
+                    bb[i] = dot(dF[i], f, n);
+                    for (int j = 0; j < mk; ++j) Nm[i + (size_t)mk * j] = dot(dF[i], dF[j], n);
+                }
             }
             double tr = 0.0;
             for (int i = 0; i < mk; ++i) tr += Nm[i + (size_t)mk * i];
@@ -1248,12 +1291,17 @@ void Problem::anderson(size_t n, double* z, FP fixedpoint, int64_t& iter, double
                 for (int j = kq + 1; j < mk; ++j) s -= M[kq + (size_t)mk * j] * x[j];
                 x[kq] = M[kq + (size_t)mk * kq] != 0.0 ? s / M[kq + (size_t)mk * kq] : 0.0;
             }
-            k_axpy(1.0, f, z, n, st);
             // z <- z + f - sum gamma_i dG_i  (the (beta-1) dF term vanishes for beta = 1)
-            for (int i = 0; i < mk; ++i) k_axpy(-x[i], dG[i], z, n, st);
+            if (fused) {
+                for (int i = 0; i < mk; ++i) t.gamma[i] = x[i];
+                launch_anderson_update(t, (long)n, st);
+            } else {
+                k_axpy(1.0, f, z, n, st);
+                for (int i = 0; i < mk; ++i) k_axpy(-x[i], dG[i], z, n, st);
+            }
         }
-        k_copy(fo, f, n, st);
-        k_copy(go, g, n, st);
+        std::swap(f, fo);
+        std::swap(g, go);
     }
     rho = rho_estimate(resid0, resid, iter);
 }
@@ -1275,8 +1323,10 @@ void Problem::livolant(size_t n, double* z, FP fixedpoint, int period, int64_t& 
         fixedpoint(g, z); ++iter;
         k_copy(f, g, n, st);
         k_axpy(-1.0, z, f, n, st);
-        const double fnorm = norm(f, n);
-        const double sc = std::max(norm(g, n), 1e-16);
+        double ff, gg;
+        dot2(f, f, g, g, n, ff, gg);
+        const double fnorm = std::sqrt(ff);
+        const double sc = std::max(std::sqrt(gg), 1e-16);
         resid = fnorm / sc;
         if (std::isnan(resid0)) resid0 = resid;
         if (resid < tol) { k_copy(z, g, n, st); conv = true; break; }
@@ -1287,7 +1337,8 @@ void Problem::livolant(size_t n, double* z, FP fixedpoint, int period, int64_t& 
             k_sub(e0, z1, z0, n, st);
             k_sub(de, g, z1, n, st);
             k_axpy(-1.0, e0, de, n, st);
-            const double se = dot(e0, de, n), sd = dot(de, de, n);
+            double se, sd;
+            dot2(e0, de, de, de, n, se, sd);
             double mu = 1.0;
             if (sd != 0.0) { mu = -se / sd; if (mu <= 0) mu = 1.0; }
             k_copy(z, g, n, st);
@@ -1347,9 +1398,10 @@ void Problem::bicgstab(size_t n, double* z, MV matvec, const double* c, int64_t&
             break;
         }
         matvec(t, s); ++iter;
-        const double tt = dot(t, t, n);
+        double tt, ts;
+        dot2(t, t, t, s, n, tt, ts);
         if (tt < tiny) break;
-        om = dot(t, s, n) / tt;
+        om = ts / tt;
         k_axpy(al, p, z, n, st);
         k_axpy(om, s, z, n, st);
         k_copy(r, s, n, st);
@@ -1398,15 +1450,31 @@ void Problem::solve_group_plain(int g, rt_group_stats& s) {
     } else {
         double* c = vec("c", n);
         T(c, nullptr);  // c = T(0)
-        k_fill(z, 0.0, n, st);
-        if (accel == RT_ACCEL_GMRES) gmres(n, z, MV, c, restart, maxit, tol, niter, resid, conv, rho, "g");
-        else bicgstab(n, z, MV, c, niter, resid, conv, rho);
+        if (accel == RT_ACCEL_GMRES) {
+            // a linear pass of the zero state without sources is zero: no need to run it (the
+            // adaptive closure's pass is not linear)
+            if (adapt) k_fill(z, 0.0, n, st);
+            gmres(n, z, MV, c, restart, maxit, tol, niter, resid, conv, rho, "g", !adapt);
+        } else {
+            k_fill(z, 0.0, n, st);
+            bicgstab(n, z, MV, c, niter, resid, conv, rho);
+        }
     }
-    // reconstruction pass 𝚽l = T(z) (sn_one_speed.jl:186)
+    // reconstruction pass 𝚽l = T(z) (sn_one_speed.jl:186), straight into the group's flux; its exit
+    // faces are not needed
     if (faithful) {
-        double* out = vec("recon", n);
-        pass_faithful(g, P64, MODE_T, z, out);
-        k_copy(d_phi + (size_t)g * Np * Nc, out, (size_t)Np * Nc, st);
+        PassDesc pd;
+        fill_geometry(pd, g);
+        pd.Mact = d_Mact64;
+        pd.qlout = d_qlout;
+        pd.phi_in = z;
+        pd.phi_rows = d_act;
+        pd.Nrows = Np;
+        pd.Drows = d_D64;
+        pd.out = d_phi + (size_t)g * Np * Nc;
+        set_csd(pd, g);
+        if (has_bc || has_ss) set_boundary(pd, g, MODE_T, z, nullptr, (size_t)Np * Nc);
+        launch_pass(pd, P64, true);
     } else {
         pass_reconstruct(g, z);
     }
@@ -1438,24 +1506,23 @@ void Problem::solve_group_mixed(int g, rt_group_stats& s) {
     bool have_az = false;  // d_psi holds the angular flux of A z at the current z
     k_fill(z, 0.0, n, st);
     if (bnorm > 0.0) {
-        k_copy(r, c, n, st);
         resid = 1.0;
         conv = false;
         auto MVlo = [&](double* out, const double* in) { pass_reduced(g, lo, MODE_IMA, in, out); };
         while (true) {
             if (resid < tol) { conv = true; break; }
             if (refs >= max_ref || niter >= maxit) break;
-            k_fill(dz, 0.0, n, st);
             int64_t it = 0;
             double rr, rh;
             bool cv;
-            gmres(n, dz, MVlo, r, restart, maxit - niter, inner_tol, it, rr, cv, rh, "m", true, true);
+            gmres(n, dz, MVlo, refs == 0 ? c : r, restart, maxit - niter, inner_tol, it, rr, cv, rh, "m", true, true);
             niter += it;
             k_axpy(1.0, dz, z, n, st);
             pass_reduced(g, P64, MODE_IMA, z, t);  // t = z - A z in FP64
             have_az = true;
-            k_sub(r, c, t, n, st);                  // r = c - (I - A) z
-            resid = norm(r, n) / bnorm;
+            launch_residual(r, c, t, (long)n, aw, ++seq, st);  // r = c - (I - A) z
+            wait_host(seq);
+            resid = std::sqrt(h_scal[0]) / bnorm;
             ++refs;
         }
     }

@@ -194,11 +194,10 @@ private:
     double* vec(const std::string& name, size_t n);
     RedWork rw{};
     double* h_scal = nullptr;   // pinned mirror of the scalar slots
+    double** d_Vptr = nullptr;  // device table of Krylov basis pointers (lockstep batches)
     ArnoldiWork aw{};           // workspace of the Arnoldi steps
     unsigned long long seq = 0; // results asked of the device so far (the pinned counter's next value)
     void wait_host(unsigned long long seq);
-    double** d_Vptr = nullptr;  // device table of Krylov basis pointers
-    double* d_y = nullptr;
 
     // passes
     void pass_faithful(int g, int prec, int mode, const double* zin, double* zout, const double* caller_q = nullptr);
@@ -218,6 +217,7 @@ private:
 
     // BLAS-1 helpers
     double dot(const double* a, const double* b, size_t n);
+    void dot2(const double* a, const double* b, const double* c, const double* d, size_t n, double& ab, double& cd);
     double norm(const double* a, size_t n) { return std::sqrt(dot(a, a, n)); }
 
     // solvers over a state of length n; pass(out, in) applies the operator

@@ -2805,14 +2805,6 @@ __global__ void scale_inv_slot_kernel(double* __restrict__ d, const double* __re
     const double a = 1.0 / h;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) d[i] = s[i] * a;
 }
-__global__ void lincomb_kernel(double* __restrict__ z, const double* const* __restrict__ V, const double* __restrict__ y, int k,
-                               size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        double v = z[i];
-        for (int t = 0; t < k; ++t) v += y[t] * V[t][i];
-        z[i] = v;
-    }
-}
 __global__ void cast_kernel(float* __restrict__ d, const double* __restrict__ s, size_t n) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) d[i] = (float)s[i];
 }
@@ -2825,9 +2817,6 @@ __global__ void scatter_rows_kernel(double* __restrict__ dst, const double* __re
     }
 }
 __global__ void set_pd_kernel(PassDesc v, PassDesc* dst) { *dst = v; }
-__global__ void set_vals_kernel(Vals32 v, double* dst, int k) {
-    if ((int)threadIdx.x < k) dst[threadIdx.x] = v.v[threadIdx.x];
-}
 // phi_all [g][p][c] -> Radiant 𝚽l[g + G*(p + Np*c)]
 // dst[g + G (p + Np (c - c0))] = src[(g Np + p) Nc + c] for the cells c0 <= c < c0 + nc
 __global__ void phi_to_radiant_kernel(double* __restrict__ dst, const double* __restrict__ src, int G, int Np, int Nc,
@@ -3729,10 +3718,6 @@ void k_scale_by_inv_slot(double* dst, const double* src, const double* scal, int
     hipLaunchKernelGGL(scale_inv_slot_kernel, dim3(grid_for(n)), dim3(256), 0, st, dst, src, scal, slot, n);
     RT_HIP(hipGetLastError());
 }
-void k_lincomb(double* z, const double* const* V, const double* y, int k, size_t n, hipStream_t st) {
-    hipLaunchKernelGGL(lincomb_kernel, dim3(grid_for(n)), dim3(256), 0, st, z, V, y, k, n);
-    RT_HIP(hipGetLastError());
-}
 void k_cast_f64_f32(float* dst, const double* src, size_t n, hipStream_t st) {
     hipLaunchKernelGGL(cast_kernel, dim3(grid_for(n)), dim3(256), 0, st, dst, src, n);
     RT_HIP(hipGetLastError());
@@ -3743,10 +3728,6 @@ void k_scatter_state(double* dst, const double* src, int rows, const int* rowmap
 }
 void k_set_pd(const PassDesc& v, PassDesc* dst, hipStream_t st) {
     hipLaunchKernelGGL(set_pd_kernel, dim3(1), dim3(1), 0, st, v, dst);
-    RT_HIP(hipGetLastError());
-}
-void k_set_vals(const Vals32& v, double* dst, int k, hipStream_t st) {
-    hipLaunchKernelGGL(set_vals_kernel, dim3(1), dim3(32), 0, st, v, dst, k);
     RT_HIP(hipGetLastError());
 }
 void k_phi_to_radiant(double* dst, const double* phi_all, int G, int Np, int Nc, int c0, int nc, hipStream_t st) {

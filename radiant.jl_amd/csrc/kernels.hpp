@@ -289,9 +289,7 @@ void k_neg_add(double* r, const double* c, size_t n, hipStream_t st);           
 // dst = src * (1/sqrt(scal[slot])) when scal[slot] > 0 (the slot holds a squared norm)
 void k_scale_by_inv_slot(double* dst, const double* src, const double* scal, int slot, size_t n, hipStream_t st);
 struct Vals32 { double v[32]; };
-void k_set_vals(const Vals32& v, double* dst, int k, hipStream_t st);   // stream-ordered small upload
 void k_set_pd(const PassDesc& v, PassDesc* dst, hipStream_t st);       // stream-ordered PassDesc upload
-void k_lincomb(double* z, const double* const* V, const double* y, int k, size_t n, hipStream_t st);
 void k_sub(double* out, const double* a, const double* b, size_t n, hipStream_t st);   // out = a - b
 void k_cast_f64_f32(float* dst, const double* src, size_t n, hipStream_t st);
 void k_scatter_state(double* dst, const double* src, int rows, const int* rowmap, int Nc, hipStream_t st);
@@ -352,6 +350,30 @@ struct ArnoldiWork {
 };
 void launch_arnoldi(const BasisTab& V, double* w, double* vnext, long n, int k, bool mgs, const ArnoldiWork& aw,
                     unsigned long long seq, hipStream_t st);
+
+// Inner products a_i . b_i of up to DOT_MAX pairs of length n, sent to the pinned results.
+constexpr int DOT_MAX = 4;
+struct DotTab { const double *a[DOT_MAX], *b[DOT_MAX]; int n; };
+void launch_dots(const DotTab& t, long n, const ArnoldiWork& aw, unsigned long long seq, hipStream_t st);
+// r = c - t, its squared norm to the pinned results
+void launch_residual(double* r, const double* c, const double* t, long n, const ArnoldiWork& aw, unsigned long long seq,
+                     hipStream_t st);
+void launch_scale_copy(double* d, const double* s, double a, long n, hipStream_t st);  // d = a s
+// z = (add ? z : 0) + sum_(i < k) y_i V_i, k <= 32
+void launch_combine(double* z, const BasisTab& V, const Vals32& y, int k, bool add, long n, hipStream_t st);
+// One Anderson iteration over a history of mk differences (the newest, formed here, last; 0 in the
+// first iteration): f = g - z, the differences, and to the pinned results f.f, z.z, g.g, dF_i . f at
+// 3 + i and dF_new . dF_i at 3 + AND_DEPTH + i; then the update z += f - sum gamma_i dG_i.
+constexpr int AND_DEPTH = 8;  // depths above go vector by vector
+struct AndersonTab {
+    const double *g, *fo, *go;
+    double *z, *f;
+    double *dF[AND_DEPTH], *dG[AND_DEPTH];
+    double gamma[AND_DEPTH];
+    int mk;
+};
+void launch_anderson(const AndersonTab& t, long n, const ArnoldiWork& aw, unsigned long long seq, hipStream_t st);
+void launch_anderson_update(const AndersonTab& t, long n, hipStream_t st);
 
 // Layout converters of the host boundary (Radiant order <-> device order).
 void k_phi_to_radiant(double* dst, const double* phi_all, int G, int Np, int Nc, int c0, int nc, hipStream_t st);

@@ -392,7 +392,164 @@ void arnoldi_km(const BasisTab& V, double* w, double* vnext, long n, int k, bool
                        p2, nb, aw.h, k, aw.host, seq);
 }
 
+// ------------------------------------------------------------------------------------------
+// Inner products a_i . b_i of up to DOT_MAX pairs in one pass, and the Anderson step.
+// ------------------------------------------------------------------------------------------
+template <int NV>
+__device__ inline void block_partials(double (&v)[NV], int nv, double* __restrict__ part) {
+    __shared__ double red[4][NV];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        if (i < nv) {  // uniform
+            const double s = wave_sum(v[i]);
+            if (lane == 63) red[wv][i] = s;
+        }
+    __syncthreads();
+    if ((int)threadIdx.x < nv)
+        part[(size_t)blockIdx.x * NV + threadIdx.x] =
+            ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x];
+}
+
+__global__ __launch_bounds__(256) void dots_kernel(const DotTab t, long n, double* __restrict__ part) {
+    double acc[DOT_MAX] = {};
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L)
+#pragma unroll
+        for (int j = 0; j < DOT_MAX; ++j)
+            if (j < t.n) acc[j] = fma(gld(t.a[j] + i), gld(t.b[j] + i), acc[j]);
+    block_partials<DOT_MAX>(acc, t.n, part);
+}
+
+// one block: the sums of nv values over nb partials, to the host
+template <int NV>
+__global__ __launch_bounds__(1024) void sums_to_host_kernel(const double* __restrict__ part, int nb, int nv, double* host,
+                                                            unsigned long long seq) {
+    __shared__ double out[64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    for (int v = wv; v < nv; v += 16) {
+        double s = 0.0;
+        for (int b = lane; b < nb; b += 64) s += part[(size_t)b * NV + v];
+        s = wave_sum(s);
+        if (lane == 63) out[v] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) to_host(host, out, nv, seq);
+}
+
+// One pass over the state for one Anderson iteration (anderson.jl:60-99): f = g - z, the new
+// differences dF = f - f_old and dG = g - g_old (not in the first iteration), and every inner
+// product the host needs: f.f, z.z, g.g, then dF_i . f and dF_new . dF_i of the history, the new
+// difference last.
+constexpr int AND_NV = 3 + 2 * AND_DEPTH;
+__global__ __launch_bounds__(256) void anderson_kernel(const AndersonTab t, long n, double* __restrict__ part) {
+    double acc[AND_NV] = {};
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
+        const double g = gld(t.g + i), z = gld(t.z + i), f = g - z;
+        gst(t.f + i, f);
+        acc[0] = fma(f, f, acc[0]);
+        acc[1] = fma(z, z, acc[1]);
+        acc[2] = fma(g, g, acc[2]);
+        if (t.mk > 0) {  // uniform
+            const double dn = f - gld(t.fo + i);
+            gst(t.dF[t.mk - 1] + i, dn);
+            gst(t.dG[t.mk - 1] + i, g - gld(t.go + i));
+#pragma unroll
+            for (int j = 0; j < AND_DEPTH; ++j)
+                if (j < t.mk) {
+                    const double d = j == t.mk - 1 ? dn : gld(t.dF[j] + i);
+                    acc[3 + j] = fma(d, f, acc[3 + j]);
+                    acc[3 + AND_DEPTH + j] = fma(dn, d, acc[3 + AND_DEPTH + j]);
+                }
+        }
+    }
+    block_partials<AND_NV>(acc, AND_NV, part);
+}
+
+// z <- z + f - sum_i gamma_i dG_i
+__global__ __launch_bounds__(256) void anderson_update_kernel(const AndersonTab t, long n) {
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
+        double z = gld(t.z + i) + gld(t.f + i);
+#pragma unroll
+        for (int j = 0; j < AND_DEPTH; ++j)
+            if (j < t.mk) z = fma(-t.gamma[j], gld(t.dG[j] + i), z);
+        gst(t.z + i, z);
+    }
+}
+
+// r = c - t with |r|^2
+__global__ __launch_bounds__(256) void residual_kernel(double* __restrict__ r, const double* __restrict__ c,
+                                                       const double* __restrict__ t, long n, double* __restrict__ part) {
+    double acc[1] = {0.0};
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
+        const double x = gld(c + i) - gld(t + i);
+        gst(r + i, x);
+        acc[0] = fma(x, x, acc[0]);
+    }
+    block_partials<1>(acc, 1, part);
+}
+
+__global__ __launch_bounds__(256) void scale_copy_kernel(double* __restrict__ d, const double* __restrict__ s, double a, long n) {
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) gst(d + i, gld(s + i) * a);
+}
+
+// z = (ADD ? z : 0) + sum_i y_i V_i
+template <bool ADD>
+__global__ __launch_bounds__(256) void combine_kernel(double* __restrict__ z, const BasisTab V, const Vals32 y, int k, long n) {
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
+        double x = ADD ? gld(z + i) : 0.0;
+#pragma unroll 8
+        for (int t = 0; t < k; ++t) x = fma(y.v[t], gld(V.p[t] + i), x);
+        gst(z + i, x);
+    }
+}
+
+int red_blocks(long n) {
+    const long b = (n + 1023) / 1024;
+    return (int)(b < 1 ? 1 : (b > ARN_BLOCKS ? ARN_BLOCKS : b));
+}
+
 }  // namespace
+
+void launch_dots(const DotTab& t, long n, const ArnoldiWork& aw, unsigned long long seq, hipStream_t st) {
+    if (t.n < 1 || t.n > DOT_MAX) throw std::runtime_error("launch_dots: pairs out of range");
+    const int nb = red_blocks(n);
+    hipLaunchKernelGGL(dots_kernel, dim3(nb), dim3(256), 0, st, t, n, aw.part);
+    hipLaunchKernelGGL((sums_to_host_kernel<DOT_MAX>), dim3(1), dim3(1024), 0, st, aw.part, nb, t.n, aw.host, seq);
+    RT_HIP(hipGetLastError());
+}
+
+void launch_residual(double* r, const double* c, const double* t, long n, const ArnoldiWork& aw, unsigned long long seq,
+                     hipStream_t st) {
+    const int nb = red_blocks(n);
+    hipLaunchKernelGGL(residual_kernel, dim3(nb), dim3(256), 0, st, r, c, t, n, aw.part);
+    hipLaunchKernelGGL((sums_to_host_kernel<1>), dim3(1), dim3(1024), 0, st, aw.part, nb, 1, aw.host, seq);
+    RT_HIP(hipGetLastError());
+}
+
+void launch_scale_copy(double* d, const double* s, double a, long n, hipStream_t st) {
+    hipLaunchKernelGGL(scale_copy_kernel, dim3(2 * red_blocks(n)), dim3(256), 0, st, d, s, a, n);
+    RT_HIP(hipGetLastError());
+}
+
+void launch_combine(double* z, const BasisTab& V, const Vals32& y, int k, bool add, long n, hipStream_t st) {
+    if (k < 0 || k > 32) throw std::runtime_error("launch_combine: vectors out of range");
+    if (add) hipLaunchKernelGGL(combine_kernel<true>, dim3(2 * red_blocks(n)), dim3(256), 0, st, z, V, y, k, n);
+    else hipLaunchKernelGGL(combine_kernel<false>, dim3(2 * red_blocks(n)), dim3(256), 0, st, z, V, y, k, n);
+    RT_HIP(hipGetLastError());
+}
+
+void launch_anderson(const AndersonTab& t, long n, const ArnoldiWork& aw, unsigned long long seq, hipStream_t st) {
+    if (t.mk < 0 || t.mk > AND_DEPTH) throw std::runtime_error("launch_anderson: depth out of range");
+    const int nb = red_blocks(n);
+    hipLaunchKernelGGL(anderson_kernel, dim3(nb), dim3(256), 0, st, t, n, aw.part);
+    hipLaunchKernelGGL((sums_to_host_kernel<AND_NV>), dim3(1), dim3(1024), 0, st, aw.part, nb, AND_NV, aw.host, seq);
+    RT_HIP(hipGetLastError());
+}
+
+void launch_anderson_update(const AndersonTab& t, long n, hipStream_t st) {
+    hipLaunchKernelGGL(anderson_update_kernel, dim3(red_blocks(n)), dim3(256), 0, st, t, n);
+    RT_HIP(hipGetLastError());
+}
 
 void launch_arnoldi(const BasisTab& V, double* w, double* vnext, long n, int k, bool mgs, const ArnoldiWork& aw,
                     unsigned long long seq, hipStream_t st) {

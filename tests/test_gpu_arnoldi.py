@@ -18,3 +18,18 @@ def test_solve_forms(oracle, cells, restart):
     print(cells, restart, rel_err(phi, ref), [s["niter"] for s in st], [s["niter"] for s in rst], flush=True)
     assert rel_err(phi, ref) < 1e-10 and all(s["converged"] for s in st)
     assert [s["niter"] for s in st] == [s["niter"] for s in rst]
+
+
+@pytest.mark.parametrize("depth", [1, 2, 8, 9])
+def test_anderson_depths(oracle, depth):
+    """The one-pass Anderson iteration (depths up to 8) and the vector-by-vector one beyond it, on a
+    solve long enough for the oldest difference to leave the history."""
+    from radiant_hip import problems, solver
+    from util import rel_err
+    p = problems.small_problem(2, dims=(9, 7), G=2, L=2, quad_order=4, seed=33, tol=1e-11, bc=[1, 1, 0, 1])
+    p.accel, p.depth = "anderson", depth
+    ref, rst = oracle.solve(p)
+    phi, st = solver.compute_flux(p)
+    print(depth, rel_err(phi, ref), [s["niter"] for s in st], [s["niter"] for s in rst], flush=True)
+    assert rel_err(phi, ref) < 1e-9 and all(s["converged"] for s in st)
+    assert max(s["niter"] for s in st) > depth + 2
