@@ -871,7 +871,7 @@ void Problem::launch_pass(PassDesc& pd, int prec, bool full_rows) {
         } else if (bfp && hog)
             launch_sweep_hog_bfp(sp, d_pd, Nd, ndims, ho_KE, ho_Kx, ho_Ky, ho_Kz, ho_fc, ho_lds(sp), d_hog, st);
         else if (bfp)
-            launch_sweep_bfp(sp, d_pd, Nd, ho_KE, ho_Kx, ho_Ky, ho_Kz, ho_fc, ho_lds(sp), st);
+            launch_sweep_bfp(sp, d_pd, Nd, ndims, ho_KE, ho_Kx, ho_Ky, ho_Kz, ho_fc, ho_lds(sp), st);
         else if (hog)
             launch_sweep_hog(sp, d_pd, Nd, ndims, ho_Kx, ho_Ky, ndims == 3 ? ho_Kz : 1, ho_fc, ho_lds(sp), d_hog, st);
         else if (ho_K && ndims == 3)

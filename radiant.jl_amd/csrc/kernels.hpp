@@ -220,7 +220,7 @@ int bfp_cell_moments(int Ke, int Kx, int Ky, int Kz, bool fc);
 int bfp_face_moments(int axis, int Ke, int Kx, int Ky, int Kz, bool fc);  // axis 0 = E, 1..3 = x, y, z
 bool sweep_bfp_supported(int ndims, int Ke, int Kx, int Ky, int Kz, bool fc);
 size_t sweep_bfp_lds_bytes(int prec, int ndims, int Nx, int Ny, int Nz, int Ke, int Kx, int Ky, int Kz, bool fc);
-void launch_sweep_bfp(int prec, const PassDesc* d_pd, int Nd, int Ke, int Kx, int Ky, int Kz, bool fc, size_t lds,
+void launch_sweep_bfp(int prec, const PassDesc* d_pd, int Nd, int ndims, int Ke, int Kx, int Ky, int Kz, bool fc, size_t lds,
                       hipStream_t st);
 // energy outflow of the slowing-down closure from a pass's angular flux (sweep-free reconstruction):
 // psiE_out = w_0 psiE_in + sum_e C_e (-1)^e w_(e+1) psi_(e, m), n = Nd * cells * fm_e entries
