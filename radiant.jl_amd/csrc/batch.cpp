@@ -585,14 +585,14 @@ void BatchSolver::launch_passes(const std::vector<int>& who, const std::vector<P
             const int sp = prec[i] == P64 ? (int)P64 : (int)P32;
             const int nd_ = P->Nd, K = P->ho_K, kx = P->ho_Kx, ky = P->ho_Ky, kz = P->ho_Kz, dims = P->ndims;
             const bool fc = P->ho_fc, bfp = P->bfp;
-            const int ke = P->ho_KE;
+            const int ke = P->ho_KE, gx = P->Nx, gy = P->Ny;
             const size_t lds = P->ho_lds(sp);
             const double hu = (double)P->Ncell * P->Nd * ((pr == PMIX && prec[i] == P64) ? 2.0 : 1.0);
             const double hb = 2.0 * (prec[i] == P64 ? 8.0 : 4.0) * (double)P->Nd * P->Nc;
             plan.push_back(timed(1, tix, hu, 0.0, hb, s, [=] {
                 if (bfp) launch_sweep_bfp(sp, one, nd_, dims, ke, kx, ky, kz, fc, lds, s);
                 else if (dims == 3) launch_sweep_3d_ho(sp, one, nd_, kx, ky, kz, fc, lds, s);
-                else if (dims == 2) launch_sweep_2d_ho(sp, one, nd_, kx, ky, fc, lds, s);
+                else if (dims == 2) launch_sweep_2d_ho(sp, one, nd_, gx, gy, kx, ky, fc, lds, s);
                 else launch_sweep_1d_ho(sp, one, nd_, K, s);
             }));
         }

@@ -877,7 +877,7 @@ void Problem::launch_pass(PassDesc& pd, int prec, bool full_rows) {
         else if (ho_K && ndims == 3)
             launch_sweep_3d_ho(sp, d_pd, Nd, ho_Kx, ho_Ky, ho_Kz, ho_fc, ho_lds(sp), st);
         else if (ho_K && ndims == 2)
-            launch_sweep_2d_ho(sp, d_pd, Nd, ho_Kx, ho_Ky, ho_fc, sweep_2d_ho_lds_bytes(sp, Nx, Ny, ho_Kx, ho_Ky), st);
+            launch_sweep_2d_ho(sp, d_pd, Nd, Nx, Ny, ho_Kx, ho_Ky, ho_fc, sweep_2d_ho_lds_bytes(sp, Nx, Ny, ho_Kx, ho_Ky), st);
         else if (ho_K)
             launch_sweep_1d_ho(sp, d_pd, Nd, ho_K, st);
         else if (sweep_kind == 0 && scan_cpl > 0 && sweep_scan_lds_bytes(sp, ndims, Nx, Ny, Nz, Nmat) <= 160 * 1024)

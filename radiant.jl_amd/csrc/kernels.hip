@@ -2189,9 +2189,11 @@ __device__ __forceinline__ void bndin_body(const PassDesc& d) {
         double v = 0.0;
         if (ss && sf[n] >= 0 && m == 0) {  // surface source of the entry face (first face moment)
             const double* q = ss + (size_t)sf[n] * d.ssrc_fs[ax] + pos;
+#pragma unroll 8
             for (int p = 0; p < Nps; ++p) v += Me[(size_t)n * Nps + p] * q[(size_t)p * np[ax]];
         }
         if (src >= 0 && bs)
+#pragma unroll 8
             for (int p = 0; p < Nps; ++p)
                 v += Me[(size_t)n * Nps + p] * bs[p + (size_t)Nps * (m + (size_t)fm[ax] * (src + 2 * pos))];
         out[j] = v;
@@ -3543,9 +3545,14 @@ static void ho2_dispatch(const PassDesc* d_pd, int Nd, int Kx, int Ky, bool fc, 
     }
 }
 
-void launch_sweep_2d_ho(int prec, const PassDesc* d_pd, int Nd, int Kx, int Ky, bool fc, size_t lds, hipStream_t st) {
+void launch_sweep_2d_ho(int prec, const PassDesc* d_pd, int Nd, int Nx, int Ny, int Kx, int Ky, bool fc, size_t lds,
+                        hipStream_t st) {
     if (Nd <= 0) return;
     if (lds > 160 * 1024) throw std::runtime_error("2D closure face moments exceed the LDS");
+    if (const int wpd = sweep_2d_pipe_waves(Nx, Ny, Kx, Ky, fc, lds)) {
+        launch_sweep_2d_pipe(prec, d_pd, Nd, Kx, Ky, fc, wpd, lds, st);
+        return;
+    }
     if (prec == P64) ho2_dispatch<double>(d_pd, Nd, Kx, Ky, fc, lds, st);
     else ho2_dispatch<float>(d_pd, Nd, Kx, Ky, fc, lds, st);
     RT_HIP(hipGetLastError());
