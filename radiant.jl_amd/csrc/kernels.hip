@@ -2819,17 +2819,6 @@ __global__ void scatter_rows_kernel(double* __restrict__ dst, const double* __re
     }
 }
 __global__ void set_pd_kernel(PassDesc v, PassDesc* dst) { *dst = v; }
-// phi_all [g][p][c] -> Radiant 𝚽l[g + G*(p + Np*c)]
-// dst[g + G (p + Np (c - c0))] = src[(g Np + p) Nc + c] for the cells c0 <= c < c0 + nc
-__global__ void phi_to_radiant_kernel(double* __restrict__ dst, const double* __restrict__ src, int G, int Np, int Nc,
-                                      int c0, int nc) {
-    const size_t tot = (size_t)G * Np * nc;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < tot; i += (size_t)gridDim.x * blockDim.x) {
-        const size_t g = i % G, r = i / G;
-        const size_t p = r % Np, c = c0 + r / Np;
-        dst[i] = src[(g * Np + p) * Nc + c];
-    }
-}
 // Flux at the cutoff energy (sn_flux.jl:213-218): out[p + Np*c] = sum_n D[p, n] psiE[n][c], the
 // directions summed in increasing order; DT is the k-major operator DT[n][p] = D[p, n].
 __global__ void cutoff_kernel(double* __restrict__ out, const double* __restrict__ DT, const double* __restrict__ psiE,
@@ -3735,11 +3724,6 @@ void k_scatter_state(double* dst, const double* src, int rows, const int* rowmap
 }
 void k_set_pd(const PassDesc& v, PassDesc* dst, hipStream_t st) {
     hipLaunchKernelGGL(set_pd_kernel, dim3(1), dim3(1), 0, st, v, dst);
-    RT_HIP(hipGetLastError());
-}
-void k_phi_to_radiant(double* dst, const double* phi_all, int G, int Np, int Nc, int c0, int nc, hipStream_t st) {
-    hipLaunchKernelGGL(phi_to_radiant_kernel, dim3(grid_for((size_t)G * Np * nc)), dim3(256), 0, st, dst, phi_all, G, Np,
-                       Nc, c0, nc);
     RT_HIP(hipGetLastError());
 }
 void k_cutoff(double* out, const double* DT, const double* psiE, int Np, int Nd, int Ncell, int K, int FE,

@@ -382,7 +382,6 @@ void launch_anderson(const AndersonTab& t, long n, const ArnoldiWork& aw, unsign
 void launch_anderson_update(const AndersonTab& t, long n, hipStream_t st);
 
 // Layout converters of the host boundary (Radiant order <-> device order).
-void k_phi_to_radiant(double* dst, const double* phi_all, int G, int Np, int Nc, int c0, int nc, hipStream_t st);
 // out[p + Np*c] = sum_n DT[n][p] psiE[n][c] (the cutoff-energy flux moments, Radiant's layout)
 // 𝚽cutoff [Np][K*cells] from the energy-face angular flux psiE [Nd][cells][FE]: the first FE of each
 // cell's K moments, the others zero
