@@ -1289,6 +1289,7 @@ __device__ __forceinline__ void sweep_line_body(const PassDesc& d, const int n, 
 // (no 0/0 in a void material), and b = 2 c1 + bias with bias = 1 instead of -1.  The exit
 // x-face of a row is then the flux after a lane's last cell, whatever the lane holds.
 // ------------------------------------------------------------------------------------------
+constexpr int LINE_PD_MAX = 8;  // rows in flight at most (its y rows are padded by them in LDS)
 constexpr unsigned BUF_OOB = 0x80000000u;  // beyond every num_records used here
 __device__ inline __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, unsigned bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
@@ -1454,15 +1455,18 @@ template <typename T, int CPL, int PD, bool BIN = false>
 __device__ __forceinline__ void sweep_line_fast_body(const PassDesc& d, const int n, unsigned char* smem) {
     const int ndims = d.ndims, Nx = d.Nx, Ny = d.Ny, Nc = d.Nc, Nmat = d.Nmat;
     const int lane = threadIdx.x;
-    T* hy2 = (T*)smem;   // [Ny]
-    T* st = hy2 + Ny;    // [Nmat]
+    T* hy2 = (T*)smem;         // [Ny + PD], rows in sweep order
+    T* st = hy2 + Ny + PD;     // [Nmat]
     const double mu = d.mu[n], eta = ndims >= 2 ? d.eta[n] : 0.0;
     // direction-uniform: the row order and the tangential 1D case (sn_1D_bte.jl:154-155)
     const int fys = __builtin_amdgcn_readfirstlane(eta >= 0 ? 1 : 0);
     const int tang = __builtin_amdgcn_readfirstlane((ndims == 1 && fabs(mu) <= 1e-10) ? 1 : 0);
     const bool fxs = mu >= 0;
     const double amu = fabs(mu);
-    for (int i = lane; i < Ny; i += 64) hy2[i] = (T)(ndims >= 2 ? 2.0 * (fabs(eta) / d.dy[i]) : 0.0);
+    for (int i = lane; i < Ny + PD; i += 64) {
+        const int j = i < Ny ? i : Ny - 1;
+        hy2[i] = (T)(ndims >= 2 ? 2.0 * (fabs(eta) / d.dy[fys ? j : Ny - 1 - j]) : 0.0);
+    }
     for (int i = lane; i < Nmat; i += 64) st[i] = (T)d.sigt[i];
     const T* psi = (const T*)d.psi + (size_t)n * Nc;
     const int* mat = d.mat;
@@ -1514,32 +1518,41 @@ __device__ __forceinline__ void sweep_line_fast_body(const PassDesc& d, const in
     T vr[PD][CPL];
     int mr[PD][CPL];
     T xr[PD];  // x-face inflow of the row in each slot (BIN)
-    // one resource per array for the whole direction (a row is a scalar byte offset), and one
-    // with num_records 0 for the rows past the grid, which load zeros and move no bytes
+    // One resource per array for the whole direction: a row is a scalar byte offset, which goes on by
+    // a constant from row to row.  A wave issues one instruction of any kind at a time, so with one
+    // wave per SIMD what the scalar unit does per row counts as much as the vector work: forming each
+    // row's offset from its index, with a second resource for the rows past the grid, was 45 of some
+    // 105 instructions per row (128 x 128 cells, 128 directions: 29.9 -> 26.0 us in FP32, 38.5 -> 34.1
+    // in FP64; the launches of a 2D batch 12% shorter).  Forming the removal and its reciprocal, or the
+    // scan's products too, one row ahead was no faster: it is the count that bounds it, not the chain.
+    // Loads past the last row repeat it (their row is not stored); stores past it go to a resource
+    // with num_records 0, which drops them.
     const auto rpsi = buf_rsrc(psi, (unsigned)Nc * (unsigned)sizeof(T)), rpsi0 = buf_rsrc(psi, 0u);
-    const auto rmat = buf_rsrc(mat, (unsigned)Nc * 4u), rmat0 = buf_rsrc(mat, 0u);
+    const auto rmat = buf_rsrc(mat, (unsigned)Nc * 4u);
     const auto rbx = buf_rsrc(bx, (unsigned)Ny * (unsigned)sizeof(T)), rbx0 = buf_rsrc(bx, 0u);
-    auto load_row = [&](int i, int jy) __attribute__((always_inline)) {
-        const int iy = row_of(jy);
-        const bool live = jy < Ny;
-        const unsigned so = (unsigned)(Nx * iy);
+    const int sd = fys ? 1 : -1, first = fys ? 0 : Ny - 1;
+    unsigned lrow = (unsigned)(first * Nx), srow = lrow, sbx = (unsigned)first;  // in cells, in rows
+    const unsigned step = (unsigned)(sd * Nx);
+    int left = Ny - 1;  // rows after the one to be loaded next
+    auto load_row = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
-            vr[i][c] = bld_s<T>(live ? rpsi : rpsi0, offT[c], so * (unsigned)sizeof(T));
-            mr[i][c] = bld_s<int>(live ? rmat : rmat0, off4[c], so * 4u);
+            vr[i][c] = bld_s<T>(rpsi, offT[c], lrow * (unsigned)sizeof(T));
+            mr[i][c] = bld_s<int>(rmat, off4[c], lrow * 4u);
         }
+        lrow += left > 0 ? step : 0u;
+        --left;
     };
 #pragma unroll
     for (int i = 0; i < PD; ++i) {
         __builtin_amdgcn_sched_barrier(0);  // issued in slot order: slot 0 is the oldest load
-        load_row(i, i);
+        load_row(i);
         if constexpr (BIN) xr[i] = (T)gld(d.bin_x + n * npx + row_of(i));
     }
     __builtin_amdgcn_sched_barrier(0);
     // one row of slot i; rv is false only for the rows past the grid in the last block
     auto solve_row = [&](int i, int jy, bool rv) __attribute__((always_inline)) {
-        const int iy = row_of(jy);
-        const T hy = hy2[iy];
+        const T hy = hy2[jy];
         T c0[CPL], c1[CPL], a[CPL], b[CPL];
         T A = (T)0, B = (T)1;
 #pragma unroll
@@ -1562,22 +1575,24 @@ __device__ __forceinline__ void sweep_line_fast_body(const PassDesc& d, const in
             // row jy + PD goes into the ring slot just freed (kept here: the scheduler would
             // otherwise sink the loads towards their first use)
             __builtin_amdgcn_sched_barrier(0);
-            load_row(i, jy + PD);
+            load_row(i);
             __builtin_amdgcn_sched_barrier(0);
         }
         affine_scan_dpp<T>(A, B);
         T fx = wave_shr_zero(A);  // the exclusive prefix, 0 in lane 0
         if constexpr (BIN) fx = fx + dpp_move<0x138, 0xF>((T)1, B) * xr[i];
-        const unsigned so = (unsigned)(Nx * iy) * (unsigned)sizeof(T);
+        const unsigned so = srow * (unsigned)sizeof(T);
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             const T p = c0[c] + c1[c] * fx;
-            bst_s(rv ? rpsi : rpsi0, offT[c], so, p);
+            bst_s(rv ? rpsi : rpsi0, offT[c], rv ? so : 0u, p);
             const T fyn = (p + p) - fy[c];
             fy[c] = rv ? fyn : fy[c];
             fx = a[c] + b[c] * fx;
         }
-        bst_s(rv ? rbx : rbx0, bxoff, (unsigned)iy * (unsigned)sizeof(T), fx);
+        bst_s(rv ? rbx : rbx0, bxoff, rv ? sbx * (unsigned)sizeof(T) : 0u, fx);
+        srow += step;
+        sbx += (unsigned)sd;
         if constexpr (BIN) xr[i] = (T)gld(d.bin_x + n * npx + row_of(jy + PD));
     };
     int r0 = 0;
@@ -3136,7 +3151,7 @@ int sweep_scan_cpl3d(int Nx) {
 
 size_t sweep_scan_lds_bytes(int prec, int ndims, int Nx, int Ny, int Nz, int Nmat) {
     const size_t es = prec == P64 ? 8 : 4;
-    if (ndims < 3) return es * ((size_t)Ny + Nmat);
+    if (ndims < 3) return es * ((size_t)Ny + LINE_PD_MAX + Nmat);
     int cpl = sweep_scan_cpl3d(Nx) & (SCAN_PAIR - 1);
     if (cpl <= 0) cpl = 8;
     const size_t rs = (size_t)cpl * ((Nx + cpl - 1) / cpl);  // slots of a face row (sweep_scan_body)
