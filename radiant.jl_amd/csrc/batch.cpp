@@ -410,9 +410,9 @@ void BatchSolver::launch_passes(const std::vector<int>& who, const std::vector<P
     // contraction one launch writes every problem's exit-face moments.
     for (int w : fpw) {
         const PassDesc* one = dpd + w;
-        const long na = (long)ps[w].P->Nact * ps[w].P->Nc;
+        const int na = ps[w].P->Nact, nc = ps[w].P->Nc;
         hipStream_t s0 = st;
-        plan.push_back([=] { launch_fp_source(one, na, s0); });
+        plan.push_back([=] { launch_fp_source(one, na, nc, s0); });
     }
     bool any_bout = false;
     int max_nb = 0;

@@ -412,11 +412,11 @@ Problem::Problem(const rt_problem_desc& d, hipStream_t stream) {
                 }
         if (has_fp(d)) {
             // angular Fokker-Planck source T[g, mat] ℳ Φ (fokker_planck_source.jl:26-36) on the
-            // active moments: ℳ row-major [Nact][Nact], T [G][Nmat]
+            // active moments: ℳ k-major [Nact][Nact], T [G][Nmat]
             fp = true;
             std::vector<double> Ma((size_t)Nact * Nact), Tg((size_t)G * Nmat);
             for (int k = 0; k < Nact; ++k)
-                for (int j = 0; j < Nact; ++j) Ma[(size_t)k * Nact + j] = d.Mfp[act[k] + (size_t)Np * act[j]];
+                for (int j = 0; j < Nact; ++j) Ma[(size_t)j * Nact + k] = d.Mfp[act[k] + (size_t)Np * act[j]];
             for (int g = 0; g < G; ++g)
                 for (int m = 0; m < Nmat; ++m) Tg[(size_t)g * Nmat + m] = d.T[g + (size_t)G * m];
             d_fpM = dalloc<double>(Ma.size()); upload(d_fpM, Ma, st);
@@ -832,8 +832,8 @@ void Problem::launch_pass(PassDesc& pd, int prec, bool full_rows) {
         have_pd = true;
     }
     if (fpsrc) {
-        if (have_pd) launch_fp_source(d_pd, (long)Nact * Nc, st);
-        else launch_fp_source_first(pd, d_pd, (long)Nact * Nc, st);
+        if (have_pd) launch_fp_source(d_pd, Nact, Nc, st);
+        else launch_fp_source_first(pd, d_pd, st);
         have_pd = true;
     }
     if (!have_pd && prec == PBF16) {

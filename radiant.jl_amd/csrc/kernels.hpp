@@ -58,7 +58,7 @@ struct PassDesc {
     double* psiE_out;
     const double* csdK;
     // angular Fokker-Planck term (null = none): T of the group per material, ℳ on the active
-    // moments [Nact][Nact], and for a pass with a non-zero state the source it builds,
+    // moments, k-major (fpM[j][k] = ℳ[k][j], [Nact][Nact]), and for a pass with a non-zero state the source it builds,
     // fpq = fp_qin + T[mat] ℳ Φ [Nact][Nc] (fp_qin: the out-of-group source, null = zero)
     const double* fpT;
     const double* fpM;
@@ -141,7 +141,7 @@ void launch_mgemm_first(int prec, const PassDesc& pd, PassDesc* d_pd, const Gemm
 void launch_mgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int ntasks, hipStream_t st, bool small = false);
 // The same for the kernels that come before the contraction.
 void launch_bndin_first(const PassDesc& pd, PassDesc* d_pd, int total, hipStream_t st);
-void launch_fp_source_first(const PassDesc& pd, PassDesc* d_pd, long n, hipStream_t st);
+void launch_fp_source_first(const PassDesc& pd, PassDesc* d_pd, hipStream_t st);
 // FP64 D contraction of one problem with the half-range moments of its exit faces (as a pass with
 // PassDesc::bout_* wants them) in one launch: the boundary work tiles follow the contraction's.
 constexpr int BND_ROWS = 32;    // half-range moments per boundary tile
@@ -191,8 +191,8 @@ void launch_bndin(const PassDesc* d_pd, int total, hipStream_t st);
 void launch_csd_source(const PassDesc* d_pd, long n, hipStream_t st);
 void launch_csd_out(const PassDesc* d_pd, long n, hipStream_t st);
 // angular Fokker-Planck source, one problem: fpq[k][c] = fp_qin[k][c] + T[mat c] sum_j ℳ[k][j]
-// phi_in[row j][c], n = Nact * Nc
-void launch_fp_source(const PassDesc* d_pd, long n, hipStream_t st);
+// phi_in[row j][c]
+void launch_fp_source(const PassDesc* d_pd, int Nact, int Nc, hipStream_t st);
 // 1D sweep of a general closure with K = PassDesc::ho_K (1..HO_KMAX) spatial moments per cell, one
 // problem, one wave per direction
 constexpr int HO_KMAX = 8;
