@@ -84,6 +84,8 @@ void BatchSolver::ensure_task_capacity() {
         ng += ntile * ((std::max(P->Nd, P->Np) + GEMM_ROWS - 1) / GEMM_ROWS);
         nsw += (size_t)P->Nd;
     }
+    // a launch below GEMM_FILL full-size tiles is cut into at most four times as many half-size ones
+    ng = std::max(ng, (size_t)4 * GEMM_FILL);
     if (ng <= cap_gemm && nsw <= cap_sweep) return;
     // the tables are rewritten every round: after the stream drains they can be replaced
     RT_CHECK(hipStreamSynchronize(st));
@@ -165,11 +167,22 @@ void BatchSolver::remove(int slot) {
     s.phase = DONE;
 }
 
-void BatchSolver::drain_pre() {
-    if (pre.empty()) return;
-    arena_off = 0;
+void BatchSolver::run_pending() {
+    if (!adds.empty()) {
+        const double* dc = stage(add_coefs.data(), add_coefs.size());
+        for (size_t a = 0; a < adds.size(); ++a) adds[a].coef = dc + 64 * a;
+        run_vecops(adds);
+        adds.clear();
+        add_coefs.clear();
+    }
     run_vecops(pre);
     pre.clear();
+}
+
+void BatchSolver::drain_pre() {
+    if (pre.empty() && adds.empty()) return;
+    arena_off = 0;
+    run_pending();
     flush();
     RT_CHECK(hipStreamSynchronize(st));
 }
@@ -445,6 +458,19 @@ void BatchSolver::launch_passes(const std::vector<int>& who, const std::vector<P
         using SKey = std::array<int, 3>;
         std::map<SKey, std::vector<int>> sweeps;
         int moff = 0, doff = 0;
+        // work-tile sizes of the group's contractions: half-size where full-size ones would leave the
+        // device idle (as for single problems; the sums keep their order, so the same bits)
+        long full_m = 0, full_d = 0;
+        for (size_t i = 0; i < who.size(); ++i)
+            if (group_of(prec[i]) == pr) {
+                const Problem* P = ps[who[i]].P;
+                const long nt = (P->Nc + GEMM_CELLS - 1) / GEMM_CELLS;
+                full_d += nt * (((full[i] ? P->Np : P->Nact) + GEMM_ROWS - 1) / GEMM_ROWS);
+                if (full[i] != 2) full_m += nt * ((P->Nd + GEMM_ROWS - 1) / GEMM_ROWS);
+            }
+        const bool sm_m = full_m < GEMM_FILL, sm_d = full_d < GEMM_FILL;
+        const int mc = sm_m ? GEMM_SMALL_CELLS : GEMM_CELLS, mr = sm_m ? GEMM_SMALL_ROWS : GEMM_ROWS;
+        const int dc = sm_d ? GEMM_SMALL_CELLS : GEMM_CELLS, drw = sm_d ? GEMM_SMALL_ROWS : GEMM_ROWS;
         std::map<SKey, int> soff;
         std::map<SKey, size_t> slds;
         std::map<SKey, double> s_upd;
@@ -466,20 +492,19 @@ void BatchSolver::launch_passes(const std::vector<int>& who, const std::vector<P
             if (group_of(prec[i]) != pr) continue;
             if (split && (prec[i] == P64) != (part == 0)) continue;
             const Problem* P = ps[who[i]].P;
-            const int ntile = (P->Nc + GEMM_CELLS - 1) / GEMM_CELLS;
-            const int nrg_m = (P->Nd + GEMM_ROWS - 1) / GEMM_ROWS;
+            const int nt_m = (P->Nc + mc - 1) / mc, nrg_m = (P->Nd + mr - 1) / mr;
             const int rows = full[i] ? P->Np : P->Nact;
-            const int nrg_d = (rows + GEMM_ROWS - 1) / GEMM_ROWS;
-            dmeta.insert(dmeta.end(), {who[i], ntile, nrg_d, doff});
-            doff += ntile * nrg_d;
+            const int nt_d = (P->Nc + dc - 1) / dc, nrg_d = (rows + drw - 1) / drw;
+            dmeta.insert(dmeta.end(), {who[i], nt_d, nrg_d, doff});
+            doff += nt_d * nrg_d;
             const double upd = (double)P->Nc * P->Nd * ((pr == PMIX && prec[i] == P64) ? 2.0 : 1.0);
             d_upd += upd;
             g_dflop += 2.0 * rows * upd;
             const double es = prec[i] == P64 ? 8.0 : 4.0, ndc = (double)P->Nd * P->Nc;
             d_by += es * ndc + 8.0 * rows * (double)P->Nc * (pds[i].zin ? 2.0 : 1.0);
             if (full[i] == 2) continue;  // contraction only: no moment->direction contraction, no sweep
-            mmeta.insert(mmeta.end(), {who[i], ntile, nrg_m, moff});
-            moff += ntile * nrg_m;
+            mmeta.insert(mmeta.end(), {who[i], nt_m, nrg_m, moff});
+            moff += nt_m * nrg_m;
             if (P->ho_K) {  // a closure above order 1: its own sweep kernel, in its pass's precision
                 ho_here.push_back(i);
                 g_upd += upd;
@@ -536,21 +561,21 @@ void BatchSolver::launch_passes(const std::vector<int>& who, const std::vector<P
         // the split launches of a mixed round: FP64 tasks [0, n64), FP32 tasks [n64, n); the
         // timing events of the pair start at the first launch and stop at the last
         auto gemm2 = [split](void (*fn)(int, const PassDesc*, const GemmTask*, int, hipStream_t, bool), int prec_,
-                             const PassDesc* pd, GemmTask* t, int n64, int n, hipStream_t s_) {
+                             const PassDesc* pd, GemmTask* t, int n64, int n, hipStream_t s_, bool small) {
             if (!split || n64 == 0 || n64 == n) {
-                fn(split ? (n64 == n ? (int)P64 : (int)P32) : prec_, pd, t, n, s_, false);
+                fn(split ? (n64 == n ? (int)P64 : (int)P32) : prec_, pd, t, n, s_, small);
                 return;
             }
             hipEvent_t a, b;
             take_launch_events(&a, &b);
             set_launch_events(a, nullptr);
-            fn(P64, pd, t, n64, s_, false);
+            fn(P64, pd, t, n64, s_, small);
             set_launch_events(nullptr, b);
-            fn(P32, pd, t + n64, n - n64, s_, false);
+            fn(P32, pd, t + n64, n - n64, s_, small);
             set_launch_events(nullptr, nullptr);
         };
         if (nm)
-            plan.push_back(timed(0, tix, g_upd, g_mflop, g_mby, s, [=] { gemm2(launch_mgemm, ps_, dpd, mg, moff64, moff, s); }));
+            plan.push_back(timed(0, tix, g_upd, g_mflop, g_mby, s, [=] { gemm2(launch_mgemm, ps_, dpd, mg, moff64, moff, s, sm_m); }));
         // slowing down (FP64 inhomogeneous passes): the energy inflow joins the angular source
         // before the sweep, and the energy outflow 2 psi - psiE_in is formed after it
         std::vector<std::pair<const PassDesc*, long>> csd_here;
@@ -600,7 +625,7 @@ void BatchSolver::launch_passes(const std::vector<int>& who, const std::vector<P
             plan.push_back([=] {
                 for (auto& c : csd_here) launch_csd_out(c.first, c.second, s);
             });
-        plan.push_back(timed(2, tix, d_upd, g_dflop, d_by, s, [=] { gemm2(launch_dgemm, ps_, dpd, dg, doff64, doff, s); }));
+        plan.push_back(timed(2, tix, d_upd, g_dflop, d_by, s, [=] { gemm2(launch_dgemm, ps_, dpd, dg, doff64, doff, s, sm_d); }));
     }
     if (fork) {
         hipStream_t s0 = st, s1 = st64;
@@ -647,8 +672,7 @@ bool BatchSolver::round() {
     // Vector operations recorded for this round run first: among them is the flux fill of a
     // group without source, whose moments the next group's out-of-group source reads.
     arena_off = 0;
-    run_vecops(pre);
-    pre.clear();
+    run_pending();
     // ---- group starts: out-of-group + volume source (sn_flux.jl:175-179)
     for (auto& s : ps) {
         if (s.phase != START) continue;
@@ -755,10 +779,7 @@ bool BatchSolver::round() {
     const auto t3 = clk::now();
     collect_times();
     // ---- host state machines
-    std::vector<double> coefs;
-    std::vector<VecItem> adds;
-    std::vector<int> add_who;
-    for (int i : who) advance(i, pre, adds, add_who, coefs);
+    for (int i : who) advance(i);
     const auto t4 = clk::now();
     host_plan += us(t0, t1);
     host_submit += us(t1, t2);
@@ -768,22 +789,9 @@ bool BatchSolver::round() {
     // the pending operations run now, so that its flux is final when round() returns.
     bool fin = false;
     for (int i : who) fin = fin || ps[i].phase == DONE;
-    if (!adds.empty() || (fin && !pre.empty())) {
-        // z += sum y V with the coefficients in the staging arena (free again after the
-        // synchronisation above)
-        arena_off = 0;
-        if (!adds.empty()) {
-            const double* dc = stage(coefs.data(), coefs.size());
-            for (size_t a = 0; a < adds.size(); ++a) adds[a].coef = dc + 64 * a;
-            run_vecops(adds);
-        }
-        if (fin) {
-            run_vecops(pre);
-            pre.clear();
-        }
-        flush();
-        RT_CHECK(hipStreamSynchronize(st));
-    }
+    // (The others, and the additions of the Arnoldi cycles that ended, wait for the next round's
+    // upload: running them here, with a synchronisation of their own, took 40 us in every third round.)
+    if (fin) drain_pre();
     return true;
 }
 
@@ -800,6 +808,8 @@ void BatchSolver::run(rt_solve_info* info) {
     timing = Timing{};
     RT_CHECK(hipEventRecord(e0, st));
     pre.clear();
+    adds.clear();
+    add_coefs.clear();
     rounds = 0;
     const int64_t graph0 = graph_updates + graph_instantiations, inst0 = graph_instantiations;
     host_plan = host_submit = host_wait = host_advance = 0;
@@ -833,8 +843,7 @@ void BatchSolver::run(rt_solve_info* info) {
 }
 
 // One step of problem i's state machine after its pass of this round.
-void BatchSolver::advance(int i, std::vector<VecItem>& pre, std::vector<VecItem>& adds, std::vector<int>& add_who,
-                          std::vector<double>& coefs) {
+void BatchSolver::advance(int i) {
     PS& s = ps[i];
     Problem* P = s.P;
     const double* slots = h_slots + (size_t)SLOTS * i;
@@ -914,13 +923,12 @@ void BatchSolver::advance(int i, std::vector<VecItem>& pre, std::vector<VecItem>
                 for (int l = a + 1; l < k; ++l) v -= h(a, l) * y[l];
                 y[a] = h(a, a) != 0.0 ? v / h(a, a) : 0.0;
             }
-            // coefficients: 64 per add item, staged by the caller (coef set there)
-            coefs.resize(64 * (adds.size() + 1), 0.0);
-            for (int a = 0; a < k; ++a) coefs[64 * adds.size() + a] = y[a];
+            // coefficients: 64 per add item, staged with it (coef set there)
+            add_coefs.resize(64 * (adds.size() + 1), 0.0);
+            for (int a = 0; a < k; ++a) add_coefs[64 * adds.size() + a] = y[a];
             VecItem it{};
             it.op = VOP_ADDMULTI; it.n = S; it.y = s.z; it.V = (const double* const*)P->d_Vptr; it.k = k;
             adds.push_back(it);
-            add_who.push_back(i);
             s.phase = RESID;
             ++s.refs;
             break;

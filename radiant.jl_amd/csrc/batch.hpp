@@ -55,6 +55,9 @@ private:
     std::vector<PS> ps;
     hipStream_t st;
     std::vector<VecItem> pre;  // vector operations to run before the next round's passes
+    std::vector<VecItem> adds;       // and before those z += sum_i y_i V_i of the finished Arnoldi cycles,
+    std::vector<double> add_coefs;   // 64 coefficients each
+    void run_pending();              // records both and forgets them
     void init_device(int capacity);
     void ensure_task_capacity();  // grows the task tables to the problems in the slots
     void start(int slot);         // resets a slot's problem to group 0
@@ -98,8 +101,7 @@ private:
                        const std::vector<int>& full);
     void run_vecops(const std::vector<VecItem>& items);
     void run_gs(const std::vector<GsItem>& items, bool update, bool norm);
-    void advance(int i, std::vector<VecItem>& pre, std::vector<VecItem>& adds, std::vector<int>& add_who,
-                 std::vector<double>& coefs);
+    void advance(int i);
     void start_arnoldi(PS& s);
 
     double host_plan = 0, host_submit = 0, host_wait = 0, host_advance = 0;  // RADIANT_HIP_HOSTPROF

@@ -588,14 +588,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 2 ? 4
 
 // FP64 and FP32 passes of different problems in one launch (PassDesc::prec per workgroup).
 template <int RT, int CT, bool MG, int NS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void contract_mixed_kernel(const PassDesc* __restrict__ pds,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RT <= 2 ? 4 : 2))) void contract_mixed_kernel(const PassDesc* __restrict__ pds,
                                                              const GemmTask* __restrict__ tasks) {
     __shared__ int rows_s[MG ? CONTRACT_KMAX : 1];
     const GemmTask tk = tasks[blockIdx.x];
     const PassDesc& d = pds[tk.prob];
     // the FP64 body keeps at most 2 stages in flight: with 4, its registers (FP64 operands and
     // accumulators) would leave room for one wave per SIMD for the FP32 passes of the launch too
-    if (d.prec == P64) contract_body<double, RT, CT, MG, (NS > 2 ? 2 : NS)>(d, tk, rows_s);
+    if (d.prec == P64) contract_body<double, RT, CT, MG, (NS > 2 && RT > 2 ? 2 : NS)>(d, tk, rows_s);
     else contract_body<float, RT, CT, MG, NS>(d, tk, rows_s);
 }
 
@@ -2959,8 +2959,8 @@ static void mgemm_any(int prec, const PassDesc* d_pd, const GemmTask* tasks, int
         if (small) launch_timed(contract_bf16_kernel<RT_SMALL, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
         else launch_timed(contract_bf16_kernel<GEMM_RT, GEMM_CT, true>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     } else if (small) {
-        if (prec == PMIX) throw std::runtime_error("launch_mgemm: half-size tiles take one precision");
-        if (first && prec == P64) launch_timed(contract_first_kernel<double, RT_SMALL, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, *first, dst, tasks);
+        if (prec == PMIX) launch_timed(contract_mixed_kernel<RT_SMALL, true, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        else if (first && prec == P64) launch_timed(contract_first_kernel<double, RT_SMALL, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, *first, dst, tasks);
         else if (first) launch_timed(contract_first_kernel<float, RT_SMALL, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, *first, dst, tasks);
         else if (prec == P64) launch_timed(contract_kernel<double, RT_SMALL, true, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
         else launch_timed(contract_kernel<float, RT_SMALL, true, SMALL_NS_M>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
@@ -3046,8 +3046,8 @@ void launch_dgemm(int prec, const PassDesc* d_pd, const GemmTask* tasks, int nta
         if (small) launch_timed(contract_bf16_kernel<RT_SMALL, false>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
         else launch_timed(contract_bf16_kernel<GEMM_RT, GEMM_CT, false>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     } else if (small) {
-        if (prec == PMIX) throw std::runtime_error("launch_dgemm: half-size tiles take one precision");
-        if (prec == P64) launch_timed(contract_kernel<double, RT_SMALL, false, SMALL_NS_D>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        if (prec == PMIX) launch_timed(contract_mixed_kernel<RT_SMALL, false, SMALL_NS_D>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
+        else if (prec == P64) launch_timed(contract_kernel<double, RT_SMALL, false, SMALL_NS_D>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
         else launch_timed(contract_kernel<float, RT_SMALL, false, SMALL_NS_D>, dim3(ntasks), dim3(256), 0, st, d_pd, tasks);
     } else {
         TuneTicket t;
