@@ -228,9 +228,11 @@ int rt_problem_pass(rt_problem *h, int32_t g, int32_t mode, const double *qlout,
  * that forbid hipMalloc), e.g. an external Krylov solver applying the transport operator to vectors
  * it keeps on the device.  qlout, z_in and z_out are DEVICE pointers (caller-allocated) in the
  * layouts of rt_problem_pass; the rows of qlout for moments without a scattering source are not
- * read.  Its temporaries live in a fixed device array of 64 MiB per GPU, held until the process
- * ends: 2*S + Np*Nx*Ny*Nz doubles (S = rt_problem_state_length) must fit in 8,388,608, else
- * RT_EINVAL.  Every call on a GPU shares that array, so calls that overlap on one GPU race.
+ * read.  The vectors are read and written in place, and z_out may be z_in.  With a Fokker-Planck
+ * or magnetic-field source, or a z_out that partly overlaps z_in, temporaries live in a fixed device
+ * array of 64 MiB per GPU, held until the process ends, which such calls share: they race when they
+ * overlap on one GPU.  Every problem must fit it: 2*S + Np*Nx*Ny*Nz doubles (S =
+ * rt_problem_state_length) in 8,388,608, else RT_EINVAL.
  * Blocking (the handle's stream is synchronised); needs a faithful FP64 handle. */
 int rt_problem_pass_device(rt_problem *h, int32_t g, int32_t mode, const double *qlout, const double *z_in,
                            double *z_out);
