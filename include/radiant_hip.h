@@ -250,6 +250,10 @@ int rt_problem_state_length(rt_problem *h, int64_t *S);
  * direction->moment (which = 1) contraction kernel at precision prec (RT_PREC_*). */
 int rt_test_contraction(int32_t which, int32_t prec, int32_t M, int32_t K, int32_t N, const double *A,
                         const double *B, double *C);
+/* Kernel-level test hook: copies phi[G][Np][Nc] (cell fastest, host) to the device and out again as
+ * Radiant's 𝚽l [Nc][Np][G] (group fastest), with the pieces written to pinned memory by kernels
+ * (way = 0) or by the copy engines (1), or without pinned memory (2). */
+int rt_test_flux_out(int32_t way, int32_t G, int32_t Np, int32_t Nc, const double *phi, double *out);
 
 /* ------------------------------------------------------------------------------------------
  * Batched solve: n independent problems advanced together (one sweep launch covers every

@@ -7,6 +7,7 @@
 #include <string>
 
 #include "engine.hpp"
+#include "flux_out.hpp"
 
 namespace {
 thread_local std::string g_last_error;
@@ -121,6 +122,12 @@ int rt_test_contraction(int32_t which, int32_t prec, int32_t M, int32_t K, int32
     if (!A || !B || !C || M < 1 || K < 1 || N < 1 || which < 0 || which > 1 || prec < 0 || prec > 2)
         return fail(RT_EINVAL, "invalid contraction test arguments");
     return guarded([&] { rt::test_contraction(which, prec, M, K, N, A, B, C); });
+}
+
+int rt_test_flux_out(int32_t way, int32_t G, int32_t Np, int32_t Nc, const double* phi, double* out) {
+    if (!phi || !out || G < 1 || Np < 1 || Nc < 1 || way < 0 || way > 2)
+        return fail(RT_EINVAL, "invalid copy-out test arguments");
+    return guarded([&] { rt::test_flux_out(way, G, Np, Nc, phi, out); });
 }
 
 int rt_autotune(int32_t mode) {

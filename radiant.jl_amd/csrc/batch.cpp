@@ -665,6 +665,7 @@ void BatchSolver::launch_passes(const std::vector<int>& who, const std::vector<P
 // One round: every unfinished problem does one pass of its current phase, then its Krylov work;
 // the host reads the scalars and advances each problem's state machine.
 bool BatchSolver::round() {
+    const DeviceUse use;
     using clk = std::chrono::steady_clock;
     auto us = [](clk::time_point a, clk::time_point b) { return std::chrono::duration<double, std::micro>(b - a).count(); };
     const int n = (int)ps.size();

@@ -1560,7 +1560,10 @@ void Problem::solve_group(int g, rt_group_stats& s) {
     if (verbose) print_group(g, s);
 }
 
+std::atomic<int> DeviceUse::count{0};
+
 void Problem::solve(rt_group_stats* stats, rt_solve_info* info) {
+    const DeviceUse use;
     const char* pe = std::getenv("RADIANT_HIP_PROFILE");
     profiling = pe && pe[0] == '1';
     ktimes = KernelTimes{};
@@ -1601,7 +1604,10 @@ void Problem::solve(rt_group_stats* stats, rt_solve_info* info) {
     }
 }
 
-void Problem::get_flux(double* phi_out, hipStream_t s) { flux_to_host(phi_out, d_phi, G, Np, Nc, s ? s : st); }
+void Problem::get_flux(double* phi_out, hipStream_t s) {
+    const FluxWay way = DeviceUse::count.load(std::memory_order_relaxed) > 0 ? FLUX_ENGINE : FLUX_LINK;
+    flux_to_host(phi_out, d_phi, G, Np, Nc, way, s ? s : st);
+}
 
 void Problem::get_flux_cutoff(double* out, hipStream_t s) {
     if (!s) s = st;
@@ -1617,6 +1623,7 @@ void Problem::get_flux_cutoff(double* out, hipStream_t s) {
 }
 
 void Problem::host_pass(int g, int mode, const double* qlout_host, const double* zin, double* zout) {
+    const DeviceUse use;
     if (g < 0 || g >= G) throw Error(RT_EINVAL, "group out of range");
     if (mode < 0 || mode > 2) throw Error(RT_EINVAL, "pass mode must be 0 (T), 1 (A) or 2 (I - A)");
     if (state_mode != RT_STATE_FAITHFUL) throw Error(RT_EINVAL, "rt_problem_pass needs a faithful FP64 handle");
@@ -1686,6 +1693,7 @@ double* noalloc_scratch(size_t* cap) {
 
 void Problem::device_pass(int g, int mode, const double* qlout_dev, const double* zin_dev, double* zout_dev,
                           double* scr, size_t cap) {
+    const DeviceUse use;
     if (g < 0 || g >= G) throw Error(RT_EINVAL, "group out of range");
     if (mode < 0 || mode > 2) throw Error(RT_EINVAL, "pass mode must be 0 (T), 1 (A) or 2 (I - A)");
     if (state_mode != RT_STATE_FAITHFUL) throw Error(RT_EINVAL, "rt_problem_pass_device needs a faithful FP64 handle");

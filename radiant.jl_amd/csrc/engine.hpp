@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <map>
 #include <string>
@@ -41,6 +42,16 @@ double inner_tol_for(int prec);
 
 // Runs one contraction kernel in isolation (test hook behind rt_test_contraction).
 void test_contraction(int which, int prec, int M, int K, int N, const double* A, const double* B, double* C);
+
+// Solves, passes and lockstep rounds under way in this process: a copy-out beside them moves its pieces
+// another way than one that has the device to itself (get_flux).
+struct DeviceUse {
+    static std::atomic<int> count;
+    DeviceUse() { count.fetch_add(1, std::memory_order_relaxed); }
+    ~DeviceUse() { count.fetch_sub(1, std::memory_order_relaxed); }
+    DeviceUse(const DeviceUse&) = delete;
+    DeviceUse& operator=(const DeviceUse&) = delete;
+};
 
 // Pass kinds of sn_inner_pass! / the GMRES matvec.
 enum PassMode { MODE_T = 0, MODE_A = 1, MODE_IMA = 2 };

@@ -1,14 +1,22 @@
 // flux_out.hip -- flux moments from the device into the caller's (pageable) memory.
 //
 // The flux lies [group][moment][cell] on the device and leaves as Radiant's [cell][moment][group].
-// Cells are outermost there, so a range of cells is one contiguous piece of the output: the range is
-// rearranged by a kernel that writes it straight into a pinned host buffer (the link's speed, without
-// a staging copy on the device), and host threads copy finished pieces into the caller's memory, whose
-// pages are usually touched there for the first time.  A ring of small pieces keeps the link and the
-// threads busy at once.
-// Bound by the link (57 GB/s measured into pinned memory).  With two 64 MiB staging buffers and threads
-// made for each: 1.41 GB of a 64^3 solve 36 ms, 119 MB 4.4 ms, twelve fluxes of 45 MB 23.5 ms; here 27.8
-// (51 GB/s), 2.9 and 16.5 ms.
+// Cells are outermost there, so a range of cells is one contiguous piece of the output.  Pieces go
+// through a ring of pinned host memory, from which host threads copy them into the caller's memory, whose
+// pages are usually touched there for the first time.  Small pieces keep the link and the threads
+// busy at once.  They reach the ring in one of two ways:
+//  - With nothing else running on the device, the kernel that rearranges a piece writes it straight
+//    into the ring: the link's speed without a staging copy.  Bound by the link (57 GB/s measured into
+//    pinned memory).  With two 64 MiB staging buffers and threads made for each: 1.41 GB of a 64^3
+//    solve 36 ms, 119 MB 4.4 ms, twelve fluxes of 45 MB 23.5 ms; here 27.8 (51 GB/s), 2.9 and 16.5 ms.
+//  - Beside other solves those kernels wait, piece by piece, behind the others' on the process's four
+//    hardware queues, and hold the queue and their CUs for as long as their stores cross the link:
+//    4.03 GB beside six solving threads took 196-206 ms and the solves fell from 122 to 82 a second
+//    (two staging buffers: 126-190 ms, 95-110 a second).  There the device rearranges 64 MiB at a
+//    time into device memory and the copy engines move the pieces: 135 ms, 119-123 solves a second.  From a
+//    server with eight requests in flight 4.03, 3.58 and 0.49 GB took 167-230, 156-227 and 23-41 ms (medians of
+//    runs; staging buffers 142-209, 107-176 and 20-38), now 148-153, 134-142 and 27-28.  Alone on the
+//    device this way is the slower one: 134 against 74 ms, as the copy engines reach 30 GB/s here.
 #include "flux_out.hpp"
 #include "engine.hpp"
 
@@ -60,7 +68,14 @@ constexpr size_t HUGE_PAGE = (size_t)2 << 20;
 constexpr size_t RING = (size_t)12 << 20;    // doubles of the ring (96 MiB pinned, held by the process)
 constexpr size_t PIECE_MAX = RING / 12;      // doubles of a piece at most (8 MiB)
 constexpr int SLOTS_MAX = 48;
-constexpr int STREAMS = 2;                   // pieces alternate, so that one drains while the next runs
+// Pieces alternate between two streams, so that one drains while the next runs.  Four were no faster for
+// the copy engines, and two more streams in the process moved a lockstep batch's own streams to other
+// hardware queues (41.1 -> 44.5 ms).
+constexpr int STREAMS = 2;
+// Device memory of a chunk that the copy engines empty while the next one is filled: 32 MiB does not
+// cover the wait of the rearranging kernel behind others' (145-172 ms where 64 MiB took 135), 128 MiB
+// is no faster.
+constexpr size_t CHUNK = (size_t)8 << 20;    // doubles
 
 // Doubles per piece: large ones keep the link busiest (2 MiB 49, 4 MiB 53, 8 MiB 55 GB/s of 57), small
 // ones let a small flux overlap its transfer with its copies.
@@ -73,7 +88,7 @@ size_t piece_size(size_t total) {
 struct Ring {
     std::mutex use;  // held by the copy-out that runs
     double* buf = nullptr;
-    hipEvent_t ev[SLOTS_MAX] = {}, ready_ev = nullptr;
+    hipEvent_t ev[SLOTS_MAX] = {}, ready_ev = nullptr, chunk_ev[2] = {};
     hipStream_t st[STREAMS] = {};
     bool tried = false;
     std::mutex mu;
@@ -89,6 +104,7 @@ struct Ring {
         bool ok = hipHostMalloc((void**)&buf, RING * sizeof(double), hipHostMallocDefault) == hipSuccess;
         for (auto& q : st) ok = ok && hipStreamCreateWithFlags(&q, hipStreamNonBlocking) == hipSuccess;
         for (auto& e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+        for (auto& e : chunk_ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
         ok = ok && hipEventCreateWithFlags(&ready_ev, hipEventDisableTiming) == hipSuccess;
         if (!ok) {
             (void)hipGetLastError();
@@ -161,70 +177,143 @@ Ring& ring() {
 }
 
 void launch_rows(double* dst, const double* src, int G, int Np, int Nc, size_t c0, size_t nc, hipStream_t st) {
-    hipLaunchKernelGGL(flux_rows_kernel, dim3((unsigned)((G * Np + TILE - 1) / TILE), (unsigned)((nc + TILE - 1) / TILE)), dim3(256),
-                       0, st, dst, src, G, Np, Nc, (int)c0, (int)nc);
+    constexpr size_t CELLS_MAX = (size_t)TILE << 15;  // a grid holds 65535 tiles along y
+    for (size_t a = 0; a < nc; a += CELLS_MAX) {
+        const size_t n = std::min(CELLS_MAX, nc - a);
+        hipLaunchKernelGGL(flux_rows_kernel, dim3((unsigned)((G * Np + TILE - 1) / TILE), (unsigned)((n + TILE - 1) / TILE)),
+                           dim3(256), 0, st, dst + a * G * Np, src, G, Np, Nc, (int)(c0 + a), (int)n);
+    }
     RT_HIP(hipGetLastError());
 }
 
-}  // namespace
-
-void flux_to_host(double* out, const double* phi, int G, int Np, int Nc, hipStream_t st) {
-    const size_t per = (size_t)G * Np;
-    Ring& r = ring();
-    std::unique_lock<std::mutex> lk(r.use);
-    const size_t piece = std::max(piece_size(per * Nc), std::min(per, PIECE_MAX));
-    if (per > piece || !r.ready()) {  // one cell's moments beyond a piece, or no pinned memory
-        lk.unlock();
-        const size_t cells = std::max<size_t>(1, std::min<size_t>(Nc, 4 * PIECE_MAX / per));
-        double* tmp = (double*)dev_alloc(cells * per * sizeof(double));
-        try {
-            for (size_t c0 = 0; c0 < (size_t)Nc; c0 += cells) {
-                const size_t nc = std::min(cells, (size_t)Nc - c0);
-                launch_rows(tmp, phi, G, Np, Nc, c0, nc, st);
-                RT_HIP(hipMemcpyAsync(out + c0 * per, tmp, nc * per * sizeof(double), hipMemcpyDeviceToHost, st));
-            }
-            RT_HIP(hipStreamSynchronize(st));
-        } catch (...) {
-            (void)hipStreamSynchronize(st);
-            dev_free(tmp);
-            throw;
+// Without pinned memory, or with one cell's moments beyond a piece: staged on the device and copied
+// into the caller's memory.
+void direct_out(double* out, const double* phi, int G, int Np, int Nc, hipStream_t st) {
+    const size_t per = (size_t)G * Np, cells = std::max<size_t>(1, std::min<size_t>(Nc, 4 * PIECE_MAX / per));
+    double* tmp = (double*)dev_alloc(cells * per * sizeof(double));
+    try {
+        for (size_t c0 = 0; c0 < (size_t)Nc; c0 += cells) {
+            const size_t nc = std::min(cells, (size_t)Nc - c0);
+            launch_rows(tmp, phi, G, Np, Nc, c0, nc, st);
+            RT_HIP(hipMemcpyAsync(out + c0 * per, tmp, nc * per * sizeof(double), hipMemcpyDeviceToHost, st));
         }
+        RT_HIP(hipStreamSynchronize(st));
+    } catch (...) {
+        (void)hipStreamSynchronize(st);
         dev_free(tmp);
-        return;
+        throw;
     }
+    dev_free(tmp);
+}
+
+// The kernels write the ring.
+void link_out(Ring& r, double* out, const double* phi, int G, int Np, int Nc, size_t piece, hipStream_t st) {
+    const size_t per = (size_t)G * Np;
     const size_t cells = std::min<size_t>(Nc, piece / per), np = (Nc + cells - 1) / cells;
     // a third of the ring is asked of the device ahead, the rest is being copied
     const size_t slots = std::min<size_t>(SLOTS_MAX, RING / piece), ahead = slots / 3;
     size_t issued = 0;
-    auto drain = [&] {
+    RT_HIP(hipEventRecord(r.ready_ev, st));
+    for (int q = 0; q < STREAMS; ++q) RT_HIP(hipStreamWaitEvent(r.st[q], r.ready_ev, 0));
+    for (size_t k = 0; k < np; ++k) {
+        // each once its slot's last piece, slots - ahead before the one waited for, is copied out
+        for (; issued < np && issued < k + ahead; ++issued) {
+            const int s = (int)(issued % slots);
+            r.wait_slot(s);
+            const size_t c0 = issued * cells;
+            hipStream_t q = r.st[issued % STREAMS];
+            launch_rows(r.buf + s * piece, phi, G, Np, Nc, c0, std::min(cells, (size_t)Nc - c0), q);
+            RT_HIP(hipEventRecord(r.ev[s], q));
+        }
+        const int s = (int)(k % slots);
+        RT_HIP(hipEventSynchronize(r.ev[s]));
+        const size_t c0 = k * cells, n = std::min(cells, (size_t)Nc - c0) * per;
+        if (np == 1 && n <= HUGE_PAGE / 4 / sizeof(double)) std::memcpy(out, r.buf + s * piece, n * sizeof(double));
+        else r.push(out + c0 * per, r.buf + s * piece, n, s);
+    }
+    r.wait_all();
+}
+
+// The copy engines write the ring, from chunks of whole pieces rearranged on the device (tmp: two of
+// them).  Nothing that waits for a copy goes onto a stream, where it would hold up the others of its
+// hardware queue: a piece is waited for on its stream, which nothing else uses, instead of by an event
+// behind it (with events 4.03 GB took 167-202 ms from the server and 191 beside the threads), and a chunk's kernel is
+// launched once the host has seen the chunk before the last emptied.
+void engine_out(Ring& r, double* out, const double* phi, int G, int Np, int Nc, size_t piece, double* tmp, hipStream_t st) {
+    const size_t per = (size_t)G * Np;
+    const size_t cells = std::min<size_t>(Nc, piece / per), np = (Nc + cells - 1) / cells;
+    const size_t slots = std::min<size_t>(SLOTS_MAX, RING / piece);
+    const size_t cp = CHUNK / piece, nch = (np + cp - 1) / cp;  // pieces per chunk, chunks
+    size_t launched = 0, issued = 0;
+    auto rearrange = [&] {  // the next chunk
+        const size_t c0 = launched * cp * cells, c1 = std::min<size_t>(Nc, c0 + cp * cells);
+        launch_rows(tmp + (launched & 1) * CHUNK, phi, G, Np, Nc, c0, c1 - c0, st);
+        RT_HIP(hipEventRecord(r.chunk_ev[launched & 1], st));
+        ++launched;
+    };
+    rearrange();
+    if (nch > 1) rearrange();
+    for (size_t k = 0; k < np; ++k) {
+        for (; issued < std::min(np, launched * cp) && issued < k + STREAMS; ++issued) {
+            const size_t c = issued / cp;
+            if (issued == c * cp) RT_HIP(hipEventSynchronize(r.chunk_ev[c & 1]));
+            const int s = (int)(issued % slots);
+            r.wait_slot(s);
+            const size_t n = std::min(cells, (size_t)Nc - issued * cells) * per;
+            RT_HIP(hipMemcpyAsync(r.buf + s * piece, tmp + (c & 1) * CHUNK + (issued - c * cp) * cells * per,
+                                  n * sizeof(double), hipMemcpyDeviceToHost, r.st[issued % STREAMS]));
+        }
+        RT_HIP(hipStreamSynchronize(r.st[k % STREAMS]));
+        const int s = (int)(k % slots);
+        const size_t c0 = k * cells, n = std::min(cells, (size_t)Nc - c0) * per;
+        r.push(out + c0 * per, r.buf + s * piece, n, s);
+        if ((k + 1) % cp == 0 && launched < nch) rearrange();  // chunk (k + 1) / cp - 1 is empty
+    }
+    r.wait_all();
+}
+
+}  // namespace
+
+void flux_to_host(double* out, const double* phi, int G, int Np, int Nc, FluxWay way, hipStream_t st) {
+    const size_t per = (size_t)G * Np, total = per * Nc;
+    Ring& r = ring();
+    std::unique_lock<std::mutex> lk(r.use);
+    // beside other work one launch for what fits a piece, as each waits its turn
+    const size_t piece = std::max(way == FLUX_ENGINE ? PIECE_MAX : piece_size(total), std::min(per, PIECE_MAX));
+    if (way == FLUX_DIRECT || per > piece || !r.ready()) {
+        lk.unlock();
+        direct_out(out, phi, G, Np, Nc, st);
+        return;
+    }
+    double* tmp = nullptr;
+    if (way == FLUX_ENGINE && total > piece) try {
+            tmp = (double*)dev_alloc(2 * CHUNK * sizeof(double));
+        } catch (const Error&) {  // no memory for the chunks: the kernels write the ring
+        }
+    try {
+        if (tmp) engine_out(r, out, phi, G, Np, Nc, piece, tmp, st);
+        else link_out(r, out, phi, G, Np, Nc, piece, st);
+    } catch (...) {
         (void)hipStreamSynchronize(st);
         for (auto q : r.st) (void)hipStreamSynchronize(q);
         r.wait_all();
-    };
-    try {
-        RT_HIP(hipEventRecord(r.ready_ev, st));
-        for (auto q : r.st) RT_HIP(hipStreamWaitEvent(q, r.ready_ev, 0));
-        for (size_t k = 0; k < np; ++k) {
-            // each once its slot's last piece, slots - ahead before the one waited for, is copied out
-            for (; issued < np && issued < k + ahead; ++issued) {
-                const int s = (int)(issued % slots);
-                r.wait_slot(s);
-                const size_t c0 = issued * cells;
-                hipStream_t q = r.st[issued % STREAMS];
-                launch_rows(r.buf + s * piece, phi, G, Np, Nc, c0, std::min(cells, (size_t)Nc - c0), q);
-                RT_HIP(hipEventRecord(r.ev[s], q));
-            }
-            const int s = (int)(k % slots);
-            RT_HIP(hipEventSynchronize(r.ev[s]));
-            const size_t c0 = k * cells, n = std::min(cells, (size_t)Nc - c0) * per;
-            if (np == 1 && n <= HUGE_PAGE / 4 / sizeof(double)) std::memcpy(out, r.buf + s * piece, n * sizeof(double));
-            else r.push(out + c0 * per, r.buf + s * piece, n, s);
-        }
-        r.wait_all();
-    } catch (...) {
-        drain();
+        dev_free(tmp);
         throw;
     }
+    dev_free(tmp);
+}
+
+void test_flux_out(int way, int G, int Np, int Nc, const double* phi, double* out) {
+    const size_t bytes = (size_t)G * Np * Nc * sizeof(double);
+    double* d = (double*)dev_alloc(bytes);
+    try {
+        RT_HIP(hipMemcpy(d, phi, bytes, hipMemcpyHostToDevice));
+        flux_to_host(out, d, G, Np, Nc, (FluxWay)way, nullptr);
+    } catch (...) {
+        dev_free(d);
+        throw;
+    }
+    dev_free(d);
 }
 
 }  // namespace rt

@@ -69,7 +69,7 @@ class ServerConfig(C.Structure):
 EXPORTS = ["rt_solve", "rt_problem_create", "rt_problem_solve", "rt_problem_get_flux", "rt_problem_destroy",
            "rt_problem_device_bytes", "rt_problem_pass", "rt_problem_state_length", "rt_solve_batch",
            "rt_server_create", "rt_server_submit", "rt_server_poll", "rt_server_cancel", "rt_server_destroy",
-           "rt_last_error", "rt_version", "rt_test_contraction", "rt_problem_kernel_times",
+           "rt_last_error", "rt_version", "rt_test_contraction", "rt_test_flux_out", "rt_problem_kernel_times",
            "rt_batch_create", "rt_batch_solve", "rt_batch_get_flux", "rt_batch_destroy", "rt_batch_kernel_times",
            "rt_autotune", "rt_autotune_report", "rt_solve_cutoff", "rt_problem_get_flux_cutoff",
            "rt_batch_get_flux_cutoff", "rt_server_poll_cutoff", "rt_problem_pass_device"]
@@ -102,6 +102,7 @@ def lib():
     L.rt_solve_batch.argtypes = [C.c_int32, C.POINTER(PD), C.POINTER(dp), C.POINTER(GS), C.POINTER(SolveInfo)]
     L.rt_problem_kernel_times.argtypes = [H, dp, lp]
     L.rt_test_contraction.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, dp, dp, dp]
+    L.rt_test_flux_out.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32, dp, dp]
     L.rt_batch_create.argtypes = [C.c_int32, C.POINTER(PD), C.POINTER(H)]
     L.rt_batch_solve.argtypes = [H, C.POINTER(GS), C.POINTER(SolveInfo)]
     L.rt_batch_get_flux.argtypes = [H, C.c_int32, dp]
