@@ -1139,7 +1139,7 @@ void Problem::gmres(size_t n, double* z, MV matvec, const double* c, int m, int6
         for (int j = 0; j < m; ++j) {
             if (iter >= maxit_) break;
             matvec(w, V[j]); ++iter;
-            if (m <= GS_KMAX || cgs) {
+            if (m <= GS_KMAX || (cgs && j < GS_KMAX)) {  // classical: in any cycle, up to the kernels' size
                 launch_arnoldi(tab, w, V[j + 1], (long)n, j + 1, !cgs, aw, ++seq, st);
                 wait_host(seq);
             } else {  // bases beyond the kernels' size: the chain of reductions, vector by vector
