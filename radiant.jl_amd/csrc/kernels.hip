@@ -3617,7 +3617,7 @@ void launch_sweep_2d_ho(int prec, const PassDesc* d_pd, int Nd, int Nx, int Ny, 
                         hipStream_t st) {
     if (Nd <= 0) return;
     if (lds > 160 * 1024) throw std::runtime_error("2D closure face moments exceed the LDS");
-    if (const int wpd = sweep_2d_pipe_waves(Nx, Ny, Kx, Ky, fc, lds)) {
+    if (const int wpd = sweep_2d_pipe_waves(prec, Nd, Nx, Ny, Kx, Ky, fc, lds)) {
         launch_sweep_2d_pipe(prec, d_pd, Nd, Kx, Ky, fc, wpd, lds, st);
         return;
     }

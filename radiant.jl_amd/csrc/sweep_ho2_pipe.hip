@@ -252,13 +252,31 @@ void pipe_dispatch(const PassDesc* d_pd, int Nd, int kx, int ky, bool fc, int wp
 
 }  // namespace
 
-// Up to 4 moments per cell (beyond that the solved columns do not fit the registers of a lane) and
-// diagonals that a workgroup's waves cover.
-int sweep_2d_pipe_waves(int Nx, int Ny, int kx, int ky, bool fc, size_t lds) {
-    const int m = Nx < Ny ? Nx : Ny, nm = fc ? kx * ky : kx + ky - 1;
-    if (nm > 4 || m > 64 * PIPE_WAVES || lds > PIPE_LDS_MAX) return 0;
+// Up to 4 moments per cell (beyond that the solved columns do not fit the registers of a lane), and
+// where the columns solved ahead pay for themselves: every cell is eliminated for 1 + kx + ky right-hand
+// sides where the barrier walk has one, by fewer groups the more waves a diagonal takes, and a CU
+// holds one or two of these workgroups where it holds four of the walk's.  Against the walk (in us, walk to
+// here, 36 to 64, 128 and 200 to 256 cells across at 128 directions unless stated):
+//  - One group (more than 256 cells): 693 -> 1317 (FP64, 257 cells of 4 moments), 572 -> 591 (FP32,
+//    300 of 2), 1823 -> 1636 (FP64, 512 of 2): the walk.
+//  - FP64, up to 3 moments: 78 -> 24, 267 -> 116, 474 -> 369, and still 85 -> 63 and 627 -> 485 at 800
+//    directions.
+//  - FP64, 4 moments: 93 -> 30, 303 -> 183, but 509 -> 602 with two groups (orders 2, 2; the others
+//    612 -> 566 and 581 -> 564, at 288 directions 946 -> 1170), and with the workgroups in rounds of 256 at
+//    128 cells 453 -> 410 for 512 directions, 563 -> 616 for 648, at 36 cells 96 -> 85 for 648 and
+//    94 -> 109 for 800.
+//  - FP32: 77 -> 21, 256 -> 102, 573 -> 423; with 5 face moments 85 -> 23, 285 -> 131, 626 -> 542, with two
+//    groups and 288 directions 590 -> 661.
+int sweep_2d_pipe_waves(int prec, int Nd, int Nx, int Ny, int kx, int ky, bool fc, size_t lds) {
+    const int m = Nx < Ny ? Nx : Ny, nm = fc ? kx * ky : kx + ky - 1, nf = kx + ky;
+    if (nm > 4 || m > 64 * PIPE_WAVES / 2 || lds > PIPE_LDS_MAX) return 0;
     int w = 1;
     while (64 * w < m) w *= 2;
+    if (prec == P64 && nm == 4) {
+        if (Nd > (w == 1 ? 768 : (w == 2 ? 512 : 256)) || (w > 2 && nf < 5)) return 0;
+    } else if (w > 2 && nf > 4 && Nd > 256) {
+        return 0;
+    }
     return w;
 }
 
