@@ -84,8 +84,8 @@ void BatchSolver::ensure_task_capacity() {
         ng += ntile * ((std::max(P->Nd, P->Np) + GEMM_ROWS - 1) / GEMM_ROWS);
         nsw += (size_t)P->Nd;
     }
-    // a launch below GEMM_FILL full-size tiles is cut into at most four times as many half-size ones
-    ng = std::max(ng, (size_t)4 * GEMM_FILL);
+    // a launch of half-size tiles holds at most so many
+    ng = std::max(ng, (size_t)std::max(GEMM_SMALL_M, GEMM_SMALL_D));
     if (ng <= cap_gemm && nsw <= cap_sweep) return;
     // the tables are rewritten every round: after the stream drains they can be replaced
     RT_CHECK(hipStreamSynchronize(st));
@@ -458,17 +458,16 @@ void BatchSolver::launch_passes(const std::vector<int>& who, const std::vector<P
         using SKey = std::array<int, 3>;
         std::map<SKey, std::vector<int>> sweeps;
         int moff = 0, doff = 0;
-        // work-tile sizes of the group's contractions: half-size where full-size ones would leave the
-        // device idle (as for single problems; the sums keep their order, so the same bits)
-        long full_m = 0, full_d = 0;
+        // work-tile sizes of the group's contractions, by the half-size tiles of all its problems (as for
+        // single problems; the sums keep their order, so the same bits)
+        long half_m = 0, half_d = 0;
         for (size_t i = 0; i < who.size(); ++i)
             if (group_of(prec[i]) == pr) {
                 const Problem* P = ps[who[i]].P;
-                const long nt = (P->Nc + GEMM_CELLS - 1) / GEMM_CELLS;
-                full_d += nt * (((full[i] ? P->Np : P->Nact) + GEMM_ROWS - 1) / GEMM_ROWS);
-                if (full[i] != 2) full_m += nt * ((P->Nd + GEMM_ROWS - 1) / GEMM_ROWS);
+                half_d += gemm_small_tiles(full[i] ? P->Np : P->Nact, P->Nc);
+                if (full[i] != 2) half_m += gemm_small_tiles(P->Nd, P->Nc);
             }
-        const bool sm_m = full_m < GEMM_FILL, sm_d = full_d < GEMM_FILL;
+        const bool sm_m = half_m <= (pr == PBF16 ? GEMM_SMALL_D : GEMM_SMALL_M), sm_d = half_d <= GEMM_SMALL_D;
         const int mc = sm_m ? GEMM_SMALL_CELLS : GEMM_CELLS, mr = sm_m ? GEMM_SMALL_ROWS : GEMM_ROWS;
         const int dc = sm_d ? GEMM_SMALL_CELLS : GEMM_CELLS, drw = sm_d ? GEMM_SMALL_ROWS : GEMM_ROWS;
         std::map<SKey, int> soff;

@@ -575,9 +575,9 @@ Problem::Problem(const rt_problem_desc& d, hipStream_t stream) {
         d_bscratch = dalloc<double>(std::max<size_t>(1, nb));
         d_pd = dalloc<PassDesc>(1);
         // ---- work tables
-        auto gemm_tasks = [&](int rows, int& ntask, bool& small) {
+        auto gemm_tasks = [&](bool m, int rows, int& ntask, bool& small) {
             std::vector<GemmTask> t;
-            small = gemm_small(rows, Nc);
+            small = gemm_small(m, precision == RT_PREC_MIXED_BF16 ? PBF16 : P64, rows, Nc);
             const int tiles = ceil_div(Nc, small ? GEMM_SMALL_CELLS : GEMM_CELLS),
                       rg = ceil_div(rows, small ? GEMM_SMALL_ROWS : GEMM_ROWS);
             for (int i = 0; i < tiles * rg; ++i) {
@@ -590,9 +590,9 @@ Problem::Problem(const rt_problem_desc& d, hipStream_t stream) {
             upload(p, t, st);
             return p;
         };
-        d_mg = gemm_tasks(Nd, n_mg, sm_mg);
-        d_dgf = gemm_tasks(Np, n_dgf, sm_dgf);
-        d_dga = gemm_tasks(Nact, n_dga, sm_dga);
+        d_mg = gemm_tasks(true, Nd, n_mg, sm_mg);
+        d_dgf = gemm_tasks(false, Np, n_dgf, sm_dgf);
+        d_dga = gemm_tasks(false, Nact, n_dga, sm_dga);
         if (state_mode == RT_STATE_FAITHFUL || has_bc) {
             bnd.rg = ceil_div(Nps, BND_ROWS);
             for (int ax = 0; ax < ndims; ++ax) bnd.cells[ax] = ceil_div((int)npos[ax], BND_CELLS);
@@ -1773,7 +1773,7 @@ void test_contraction(int which, int prec, int M, int K, int N, const double* A,
         std::memset(&pd, 0, sizeof(pd));
         pd.Nc = N; pd.Nmat = 1; pd.mat = dmat; pd.sigw = dsig;
         std::vector<GemmTask> t;
-        const bool small = gemm_small(M, N);
+        const bool small = gemm_small(which == 0, prec, M, N);
         for (int r = 0; r < ceil_div(M, small ? GEMM_SMALL_ROWS : GEMM_ROWS); ++r)
             for (int i = 0; i < ceil_div(N, small ? GEMM_SMALL_CELLS : GEMM_CELLS); ++i) t.push_back({0, i, r, 0});
         GemmTask* dt = (GemmTask*)al(t.size() * sizeof(GemmTask));

@@ -261,16 +261,29 @@ constexpr int GEMM_RT = 4;                      // 16-row MFMA tiles per wave
 constexpr int GEMM_CT = 4;                      // 16-cell MFMA tiles per wave
 constexpr int GEMM_ROWS = 16 * GEMM_RT;         // rows per work tile
 constexpr int GEMM_CELLS = 4 * 16 * GEMM_CT;    // cells per work tile (4 waves)
-// Problems whose work tiles of that size would fill less than one round of two workgroups per CU
-// take tiles of half the rows and half the cells (the sums keep their order, so the same bits):
-// four times the waves in flight, each with its operands reused half as often, which the L2 covers.
-// D of 128 moments, 128 directions, 16384 cells in FP64 30 -> 24 us, of 36 moments 23 -> 12 us; FP32 M and
-// D of a 128 x 128 plane 12 and 18 -> 11 and 11 us, of a 24 x 26 x 21 box 11 and 11 -> 7 and 6 us.
+// Small problems take tiles of half the rows and half the cells (the sums keep their order, so the
+// same bits): four times the waves in flight, each with its operands reused half as often, which the L2
+// covers up to a point.  They are taken while they number at most two workgroups per CU in M (three where
+// a full-size tile would be half padding), which reads its operands from three arrays and writes the larger
+// one, and six in D.  Full-size -> half-size tiles, in us, by the number of the latter, 128 directions, L = 1
+// and 5:
+//  - M in FP64: 256 9 -> 7 and 15 -> 10, 456 10 -> 10 and 16 -> 14; beyond 516 9 -> 11 and 16 -> 17, 808 10 -> 14 and
+//    16 -> 22, 1664 16 -> 22 and 28 -> 37; in FP32 1664 12 -> 17 and 20 -> 28; 32 directions 706 12 -> 12 and
+//    18 -> 17, 960 13 -> 15 and 19 -> 21.
+//  - D in FP64: 256 28 -> 13, 584 29 -> 23, 1160 47 -> 39; beyond 1664 54 -> 54, 1968 57 -> 61.
+//  - M + D in FP64 with both rules against full-size tiles, and against half-size ones in both: 584 45 -> 40
+//    (41), 1160 71 -> 62 (65), 1664 80 -> 79 (90); in FP32 31 -> 25 (27), 38 -> 36 (38), 40 -> 42 (49).
+//  - M in BF16 goes by the limit of D: 516 15 -> 12 and 18 -> 17, 808 17 -> 17 and 18 -> 22, 1160 26 -> 19 and 30 -> 26;
+//    beyond 1664 25 -> 24 and 30 -> 35; 32 directions 960 22 -> 17.
 constexpr int GEMM_SMALL_RT = 2, GEMM_SMALL_CT = 2;
 constexpr int GEMM_SMALL_ROWS = 16 * GEMM_SMALL_RT, GEMM_SMALL_CELLS = 4 * 16 * GEMM_SMALL_CT;
-constexpr int GEMM_FILL = 512;
-inline bool gemm_small(int rows, int Nc) {
-    return (long)((rows + GEMM_ROWS - 1) / GEMM_ROWS) * ((Nc + GEMM_CELLS - 1) / GEMM_CELLS) < GEMM_FILL;
+constexpr long GEMM_SMALL_M = 512, GEMM_SMALL_M32 = 768, GEMM_SMALL_D = 1536;
+inline long gemm_small_tiles(int rows, int Nc) {
+    return (long)((rows + GEMM_SMALL_ROWS - 1) / GEMM_SMALL_ROWS) * ((Nc + GEMM_SMALL_CELLS - 1) / GEMM_SMALL_CELLS);
+}
+inline bool gemm_small(bool m, int prec, int rows, int Nc) {
+    return gemm_small_tiles(rows, Nc) <=
+           (!m || prec == PBF16 ? GEMM_SMALL_D : (rows <= GEMM_SMALL_ROWS ? GEMM_SMALL_M32 : GEMM_SMALL_M));
 }
 constexpr int CONTRACT_KMAX = 1024;             // active moments at most (row map held in LDS)
 

@@ -15,6 +15,10 @@ def _problem(form):
         return P.small_problem(1, N=5, G=2, L=3, quad_order=6, seed=1)
     if form == "slab257":  # one column past a work tile
         return P.small_problem(1, N=257, G=2, L=7, quad_order=16, seed=2)
+    if form == "plane450":  # full-size tiles in M and D, the last ones ragged
+        return P.small_problem(2, dims=(450, 441), G=1, L=1, quad_order=2, seed=9)
+    if form == "plane130":  # full-size tiles in M, half-size in D
+        return P.small_problem(2, dims=(130, 127), G=1, L=3, quad_order=8, seed=10, bc=[1, 0, 0, 1])
     if form == "plane72":  # 72 moments: a second, ragged row group
         return P.small_problem(2, dims=(17, 16), G=2, L=3, quad_order=6, seed=3)
     if form == "box48":
@@ -33,7 +37,7 @@ def _problem(form):
     return p
 
 
-@pytest.mark.parametrize("form", ["slab1", "slab257", "plane72", "box48", "reflected", "closure", "fokker-planck"])
+@pytest.mark.parametrize("form", ["slab1", "slab257", "plane130", "plane450", "plane72", "box48", "reflected", "closure", "fokker-planck"])
 def test_caller_layout_forms(form):
     from test_zz_no_alloc import _Dev
     from radiant_hip import _lib, solver
