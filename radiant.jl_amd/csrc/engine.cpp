@@ -1089,9 +1089,9 @@ static double rho_estimate(double r0, double r, int64_t it) {  // krylov_state.j
 }
 
 // tools/gmres.jl:35-133 -- restarted GMRES(m), modified Gram-Schmidt, Givens rotations.
-// The host reads one H column per Arnoldi step (launch_arnoldi).  Two options
-// serve: zero_guess (z stands for zero and need not be set; the first residual is c without a pass) and
-// cgs (classical instead of modified Gram-Schmidt).
+// The host reads one H column per Arnoldi step (launch_arnoldi).  Two options: zero_guess (z stands for
+// zero and need not be set; the first residual is c without a pass) and cgs (classical instead of
+// modified Gram-Schmidt).
 template <class MV>
 void Problem::gmres(size_t n, double* z, MV matvec, const double* c, int m, int64_t maxit_, double tol_,
                     int64_t& iter, double& resid, bool& conv, double& rho, const std::string& tag, bool zero_guess,
@@ -1660,8 +1660,9 @@ void Problem::host_pass(int g, int mode, const double* qlout_host, const double*
 // ---- allocation-free pass (rt_problem_pass_device) ----
 // Scratch of the allocation-free pass: the input and output states in the engine's moment-major
 // layout and the out-of-group source, 2 S + Np Nc doubles at most NOALLOC_DOUBLES.  Every device
-// holds its own copy until the process ends; every call on a device shares it, so calls that
-// overlap on one device race.  Host code reaches it only through the address hipGetSymbolAddress
+// holds its own copy until the process ends; the calls that need it (device_pass: sources that read whole
+// moment rows, an output that partly overlaps the input) share it and race when they overlap on one
+// device.  Host code reaches it only through the address hipGetSymbolAddress
 // gives for the device (the array's name is a host-side stand-in, not a device address).
 static constexpr size_t NOALLOC_DOUBLES = (size_t)8 << 20;  // 64 MiB
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];

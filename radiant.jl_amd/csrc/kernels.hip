@@ -2886,17 +2886,6 @@ __global__ void scale_inv_slot_kernel(double* __restrict__ d, const double* __re
     const double a = 1.0 / h;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) d[i] = s[i] * a;
 }
-__global__ void cast_kernel(float* __restrict__ d, const double* __restrict__ s, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) d[i] = (float)s[i];
-}
-__global__ void scatter_rows_kernel(double* __restrict__ dst, const double* __restrict__ src, int rows, const int* __restrict__ map,
-                                    int Nc) {
-    const size_t tot = (size_t)rows * Nc;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < tot; i += (size_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / Nc), c = (int)(i % Nc);
-        dst[(size_t)map[r] * Nc + c] = src[i];
-    }
-}
 __global__ void set_pd_kernel(PassDesc v, PassDesc* dst) { *dst = v; }
 // Flux at the cutoff energy (sn_flux.jl:213-218): out[p + Np*c] = sum_n D[p, n] psiE[n][c], the
 // directions summed in increasing order; DT is the k-major operator DT[n][p] = D[p, n].
@@ -3792,14 +3781,6 @@ void k_sub(double* out, const double* a, const double* b, size_t n, hipStream_t 
 }
 void k_scale_by_inv_slot(double* dst, const double* src, const double* scal, int slot, size_t n, hipStream_t st) {
     hipLaunchKernelGGL(scale_inv_slot_kernel, dim3(grid_for(n)), dim3(256), 0, st, dst, src, scal, slot, n);
-    RT_HIP(hipGetLastError());
-}
-void k_cast_f64_f32(float* dst, const double* src, size_t n, hipStream_t st) {
-    hipLaunchKernelGGL(cast_kernel, dim3(grid_for(n)), dim3(256), 0, st, dst, src, n);
-    RT_HIP(hipGetLastError());
-}
-void k_scatter_state(double* dst, const double* src, int rows, const int* rowmap, int Nc, hipStream_t st) {
-    hipLaunchKernelGGL(scatter_rows_kernel, dim3(grid_for((size_t)rows * Nc)), dim3(256), 0, st, dst, src, rows, rowmap, Nc);
     RT_HIP(hipGetLastError());
 }
 void k_set_pd(const PassDesc& v, PassDesc* dst, hipStream_t st) {

@@ -310,8 +310,6 @@ void k_scale_by_inv_slot(double* dst, const double* src, const double* scal, int
 struct Vals32 { double v[32]; };
 void k_set_pd(const PassDesc& v, PassDesc* dst, hipStream_t st);       // stream-ordered PassDesc upload
 void k_sub(double* out, const double* a, const double* b, size_t n, hipStream_t st);   // out = a - b
-void k_cast_f64_f32(float* dst, const double* src, size_t n, hipStream_t st);
-void k_scatter_state(double* dst, const double* src, int rows, const int* rowmap, int Nc, hipStream_t st);
 
 // Batched helpers (one launch serves every problem of a batch).
 enum VecOpCode { VOP_FILL = 0, VOP_COPY = 1, VOP_SCALE_COPY = 2, VOP_NORMALIZE = 3, VOP_SUB = 4, VOP_SUBMULTI = 5,

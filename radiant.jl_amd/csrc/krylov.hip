@@ -277,8 +277,8 @@ __global__ __launch_bounds__(256) void arn_normalise_kernel(const double* __rest
     for (long i = blockIdx.x * 256L + tid; i < n; i += gridDim.x * 256L) gst(vnext + i, gld(w + i) * a);
 }
 
-// The whole step in one workgroup for short vectors (n <= ARN_SMALL): w stays in registers and the
-// basis, a few hundred kB, is read from the L2.
+// The whole step in one workgroup for short vectors (at most 1024 * ARN_SMALL_E values, ARN_SMALL_READS
+// of the basis): w stays in registers and the basis, a few hundred kB, is read from the L2.
 constexpr int ARN_SMALL_E = 8;
 template <bool MGS>
 __global__ __launch_bounds__(1024) void arn_small_kernel(const BasisTab V, double* __restrict__ w, double* __restrict__ vnext,

@@ -111,19 +111,17 @@ __global__ __launch_bounds__(256) void sweep_bfp_kernel(const PassDesc* __restri
     const size_t Ncell = (size_t)Nx * Ny * Nz;
     // face moments in LDS, or in this direction's slice of hoface (the waves of the workgroup share
     // one CU, so __syncthreads orders their device-memory writes and reads as it does for LDS)
-    const size_t nface = (size_t)Ny * Nz * F0 + (nd >= 2 ? (size_t)Nx * Nz * F1 : 0) + (nd >= 3 ? (size_t)Nx * Ny * F2 : 0);
+    const size_t nface = (size_t)Ny * Nz * F0 + (size_t)Nx * Nz * F1 + (nd >= 3 ? (size_t)Nx * Ny * F2 : 0);
     T* FX = d.hoface ? (T*)d.hoface + (size_t)n * nface : (T*)smem;  // [Ny*Nz][F0]
-    T* FY = FX + (size_t)Ny * Nz * F0;                    // [Nx*Nz][F1] (2D, 3D)
-    T* FZ = FY + (nd >= 2 ? (size_t)Nx * Nz * F1 : 0);    // [Nx*Ny][F2] (3D)
-    const double om[3] = {d.mu[n], nd >= 2 ? d.eta[n] : 0.0, nd >= 3 ? d.xi[n] : 0.0};
-    const bool tang = nd == 1 && fabs(om[0]) <= 1e-10;
+    T* FY = FX + (size_t)Ny * Nz * F0;                    // [Nx*Nz][F1]
+    T* FZ = FY + (size_t)Nx * Nz * F1;                    // [Nx*Ny][F2] (3D)
+    const double om[3] = {d.mu[n], d.eta[n], nd >= 3 ? d.xi[n] : 0.0};
     const int K3[3] = {KX, KY, KZ};
     T s[3], w[3][KM + 1], we[KM + 1], Cc[KM + 1], sp[3][KM], sn[3][KM], pe[KM];
     const double* ws[3] = {d.ho_om, d.ho_omy, d.ho_omz};
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         s[a] = om[a] > 0 ? T(1) : (om[a] < 0 ? T(-1) : T(0));
-        if (a == 0 && tang) s[a] = T(1);
 #pragma unroll
         for (int k = 0; k <= KM; ++k) w[a][k] = k <= K3[a] ? (T)ws[a][k] : T(0);
 #pragma unroll
@@ -142,8 +140,7 @@ __global__ __launch_bounds__(256) void sweep_bfp_kernel(const PassDesc* __restri
     const double* Ein = d.psiE_in ? d.psiE_in + (size_t)n * Ncell * FE : nullptr;
     double* Eout = d.psiE_out ? d.psiE_out + (size_t)n * Ncell * FE : nullptr;
     for (int i = tid; i < Ny * Nz * F0; i += nt) FX[i] = d.bin_x ? (T)d.bin_x[(size_t)n * Ny * Nz * F0 + i] : T(0);
-    if (nd >= 2)
-        for (int i = tid; i < Nx * Nz * F1; i += nt) FY[i] = d.bin_y ? (T)d.bin_y[(size_t)n * Nx * Nz * F1 + i] : T(0);
+    for (int i = tid; i < Nx * Nz * F1; i += nt) FY[i] = d.bin_y ? (T)d.bin_y[(size_t)n * Nx * Nz * F1 + i] : T(0);
     if (nd >= 3)
         for (int i = tid; i < Nx * Ny * F2; i += nt) FZ[i] = d.bin_z ? (T)d.bin_z[(size_t)n * Nx * Ny * F2 + i] : T(0);
     __syncthreads();
@@ -155,17 +152,17 @@ __global__ __launch_bounds__(256) void sweep_bfp_kernel(const PassDesc* __restri
             if (kz < 0 || kz >= Nz) continue;
             const int ix = fw[0] ? kx : Nx - 1 - kx, iy = fw[1] ? ky : Ny - 1 - ky, iz = fw[2] ? kz : Nz - 1 - kz;
             const size_t c = (size_t)ix + (size_t)Nx * (iy + (size_t)Ny * iz);
-            const T h[3] = {tang ? T(0) : (T)(fabs(om[0]) / d.dx[ix]), nd >= 2 ? (T)(fabs(om[1]) / d.dy[iy]) : T(0),
+            const T h[3] = {(T)(fabs(om[0]) / d.dx[ix]), (T)(fabs(om[1]) / d.dy[iy]),
                             nd >= 3 ? (T)(fabs(om[2]) / d.dz[iz]) : T(0)};
             const int m = d.mat[c * NM];
             const T St = (T)d.sigt[m];
             const T Sm = (T)d.csdS[2 * m], Sp = (T)d.csdS[2 * m + 1];
             const T Sv[2] = {(Sm + Sp) / T(2), (Sm - Sp) / (T(2) * sq3)};
-            T zero[F1 > F2 ? F1 : F2];  // the faces of the axes a 1D or 2D problem lacks
+            T zero[F2];  // the z faces a 2D problem lacks
 #pragma unroll
-            for (int k = 0; k < (F1 > F2 ? F1 : F2); ++k) zero[k] = T(0);
+            for (int k = 0; k < F2; ++k) zero[k] = T(0);
             T* fx = FX + ((size_t)iy + (size_t)Ny * iz) * F0;
-            T* fy = nd >= 2 ? FY + ((size_t)ix + (size_t)Nx * iz) * F1 : zero;
+            T* fy = FY + ((size_t)ix + (size_t)Nx * iz) * F1;
             T* fz = nd >= 3 ? FZ + ((size_t)ix + (size_t)Nx * iy) * F2 : zero;
             T fe[FE];
 #pragma unroll
@@ -212,7 +209,7 @@ __global__ __launch_bounds__(256) void sweep_bfp_kernel(const PassDesc* __restri
                 }
                 T r = psi[(size_t)ii + NM * c];
                 r -= Cc[a] * h[0] * (sp[0][a] * w[0][0] - sn[0][a]) * fx[H::index(e, a, b, cz, 1)];
-                if (nd >= 2) r -= Cc[b] * h[1] * (sp[1][b] * w[1][0] - sn[1][b]) * fy[H::index(e, a, b, cz, 2)];
+                r -= Cc[b] * h[1] * (sp[1][b] * w[1][0] - sn[1][b]) * fy[H::index(e, a, b, cz, 2)];
                 if (nd >= 3) r -= Cc[cz] * h[2] * (sp[2][cz] * w[2][0] - sn[2][cz]) * fz[H::index(e, a, b, cz, 3)];
                 r -= Cc[e] * (pe[e] * Sp * we[0] - Sm) * fe[H::index(e, a, b, cz, 0)];
                 q[ii] = r;
@@ -255,7 +252,7 @@ __global__ __launch_bounds__(256) void sweep_bfp_kernel(const PassDesc* __restri
 #pragma unroll
             for (int k = 0; k < F0; ++k) ox[k] = w[0][0] * fx[k];
 #pragma unroll
-            for (int k = 0; k < F1; ++k) oy[k] = nd >= 2 ? w[1][0] * fy[k] : T(0);
+            for (int k = 0; k < F1; ++k) oy[k] = w[1][0] * fy[k];
 #pragma unroll
             for (int k = 0; k < F2; ++k) oz[k] = nd >= 3 ? w[2][0] * fz[k] : T(0);
 #pragma unroll
@@ -275,12 +272,10 @@ __global__ __launch_bounds__(256) void sweep_bfp_kernel(const PassDesc* __restri
                 oz[H::index(e, a, b, cz, 3)] += Cc[cz] * sp[2][cz] * w[2][cz + 1] * v;
                 oe[H::index(e, a, b, cz, 0)] += Cc[e] * pe[e] * we[e + 1] * v;
             }
-            if (!tang)
 #pragma unroll
-                for (int k = 0; k < F0; ++k) fx[k] = ox[k];
-            if (nd >= 2)
+            for (int k = 0; k < F0; ++k) fx[k] = ox[k];
 #pragma unroll
-                for (int k = 0; k < F1; ++k) fy[k] = oy[k];
+            for (int k = 0; k < F1; ++k) fy[k] = oy[k];
             if (nd >= 3)
 #pragma unroll
                 for (int k = 0; k < F2; ++k) fz[k] = oz[k];
@@ -292,7 +287,7 @@ __global__ __launch_bounds__(256) void sweep_bfp_kernel(const PassDesc* __restri
     }
     if (d.bx)
         for (int i = tid; i < Ny * Nz * F0; i += nt) ((T*)d.bx)[(size_t)n * Ny * Nz * F0 + i] = FX[i];
-    if (nd >= 2 && d.by)
+    if (d.by)
         for (int i = tid; i < Nx * Nz * F1; i += nt) ((T*)d.by)[(size_t)n * Nx * Nz * F1 + i] = FY[i];
     if (nd >= 3 && d.bz)
         for (int i = tid; i < Nx * Ny * F2; i += nt) ((T*)d.bz)[(size_t)n * Nx * Ny * F2 + i] = FZ[i];
