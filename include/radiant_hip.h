@@ -252,8 +252,9 @@ int rt_test_contraction(int32_t which, int32_t prec, int32_t M, int32_t K, int32
                         const double *B, double *C);
 /* Kernel-level test hook: copies phi[G][Np][Nc] (cell fastest, host) to the device and out again as
  * Radiant's 𝚽l [Nc][Np][G] (group fastest), with the pieces written to pinned memory by kernels
- * (way = 0) or by the copy engines (1), or without pinned memory (2). */
-int rt_test_flux_out(int32_t way, int32_t G, int32_t Np, int32_t Nc, const double *phi, double *out);
+ * (way = 0) or by the copy engines from two blocks of chunk doubles on the device (1), or without
+ * pinned memory (2). */
+int rt_test_flux_out(int32_t way, int32_t G, int32_t Np, int32_t Nc, const double *phi, int64_t chunk, double *out);
 
 /* ------------------------------------------------------------------------------------------
  * Batched solve: n independent problems advanced together (one sweep launch covers every

@@ -124,10 +124,10 @@ int rt_test_contraction(int32_t which, int32_t prec, int32_t M, int32_t K, int32
     return guarded([&] { rt::test_contraction(which, prec, M, K, N, A, B, C); });
 }
 
-int rt_test_flux_out(int32_t way, int32_t G, int32_t Np, int32_t Nc, const double* phi, double* out) {
-    if (!phi || !out || G < 1 || Np < 1 || Nc < 1 || way < 0 || way > 2)
+int rt_test_flux_out(int32_t way, int32_t G, int32_t Np, int32_t Nc, const double* phi, int64_t chunk, double* out) {
+    if (!phi || !out || G < 1 || Np < 1 || Nc < 1 || way < 0 || way > 2 || chunk < 0)
         return fail(RT_EINVAL, "invalid copy-out test arguments");
-    return guarded([&] { rt::test_flux_out(way, G, Np, Nc, phi, out); });
+    return guarded([&] { rt::test_flux_out(way, G, Np, Nc, phi, (size_t)chunk, out); });
 }
 
 int rt_autotune(int32_t mode) {

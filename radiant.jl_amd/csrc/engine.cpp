@@ -1606,7 +1606,12 @@ void Problem::solve(rt_group_stats* stats, rt_solve_info* info) {
 
 void Problem::get_flux(double* phi_out, hipStream_t s) {
     const FluxWay way = DeviceUse::count.load(std::memory_order_relaxed) > 0 ? FLUX_ENGINE : FLUX_LINK;
-    flux_to_host(phi_out, d_phi, G, Np, Nc, way, s ? s : st);
+    // the angular fluxes of the last passes are scratch once the solve is over; a mixed solve keeps two
+    const size_t n = (size_t)Nd * Nc;
+    const auto c = pool.find("psi_c#" + std::to_string(n));
+    FluxScratch scratch{{(double*)d_psi, (double*)d_psi + n / 2}, n / 2};
+    if (c != pool.end()) scratch = {{(double*)d_psi, c->second}, n};
+    flux_to_host(phi_out, d_phi, G, Np, Nc, way, scratch, s ? s : st);
 }
 
 void Problem::get_flux_cutoff(double* out, hipStream_t s) {

@@ -15,7 +15,7 @@
 //    (two staging buffers: 126-190 ms, 95-110 a second).  There the device rearranges 64 MiB at a
 //    time into device memory and the copy engines move the pieces: 135 ms, 119-123 solves a second.  From a
 //    server with eight requests in flight 4.03, 3.58 and 0.49 GB took 167-230, 156-227 and 23-41 ms (medians of
-//    runs; staging buffers 142-209, 107-176 and 20-38), now 148-153, 134-142 and 27-28.  Alone on the
+//    runs; staging buffers 142-209, 107-176 and 20-38), now 148-155, 134-142 and 27-31.  Alone on the
 //    device this way is the slower one: 134 against 74 ms, as the copy engines reach 30 GB/s here.
 #include "flux_out.hpp"
 #include "engine.hpp"
@@ -72,10 +72,11 @@ constexpr int SLOTS_MAX = 48;
 // the copy engines, and two more streams in the process moved a lockstep batch's own streams to other
 // hardware queues (41.1 -> 44.5 ms).
 constexpr int STREAMS = 2;
-// Device memory of a chunk that the copy engines empty while the next one is filled: 32 MiB does not
-// cover the wait of the rearranging kernel behind others' (145-172 ms where 64 MiB took 135), 128 MiB
-// is no faster.
-constexpr size_t CHUNK = (size_t)8 << 20;    // doubles
+// A chunk that the copy engines empty while the next one is filled, in the scratch that the caller lends:
+// 32 MiB does not cover the wait of the rearranging kernel behind others' (145-172 ms where 64 MiB took
+// 135; 0.49 GB in chunks of 20 MiB 28-47 ms, of 41 MiB 30-31), 128 MiB is no faster.
+constexpr size_t CHUNK_MAX = (size_t)8 << 20;    // doubles
+constexpr size_t CHUNK_MIN = PIECE_MAX / 8;      // below 1 MiB the copies' own cost counts
 
 // Doubles per piece: large ones keep the link busiest (2 MiB 49, 4 MiB 53, 8 MiB 55 GB/s of 57), small
 // ones let a small flux overlap its transfer with its copies.
@@ -234,20 +235,21 @@ void link_out(Ring& r, double* out, const double* phi, int G, int Np, int Nc, si
     r.wait_all();
 }
 
-// The copy engines write the ring, from chunks of whole pieces rearranged on the device (tmp: two of
-// them).  Nothing that waits for a copy goes onto a stream, where it would hold up the others of its
-// hardware queue: a piece is waited for on its stream, which nothing else uses, instead of by an event
-// behind it (with events 4.03 GB took 167-202 ms from the server and 191 beside the threads), and a chunk's kernel is
-// launched once the host has seen the chunk before the last emptied.
-void engine_out(Ring& r, double* out, const double* phi, int G, int Np, int Nc, size_t piece, double* tmp, hipStream_t st) {
+// The copy engines write the ring, from chunks of whole pieces rearranged on the device (two of at most
+// chunk doubles, in the scratch).  Nothing that waits for a copy goes onto a stream, where it would hold up
+// the others of its hardware queue: a piece is waited for on its stream, which nothing else uses, instead
+// of by an event behind it (with events 4.03 GB took 167-202 ms from the server and 191 beside the
+// threads), and a chunk's kernel is launched once the host has seen the chunk before the last emptied.
+void engine_out(Ring& r, double* out, const double* phi, int G, int Np, int Nc, size_t piece, const FluxScratch& tmp,
+                size_t chunk, hipStream_t st) {
     const size_t per = (size_t)G * Np;
     const size_t cells = std::min<size_t>(Nc, piece / per), np = (Nc + cells - 1) / cells;
     const size_t slots = std::min<size_t>(SLOTS_MAX, RING / piece);
-    const size_t cp = CHUNK / piece, nch = (np + cp - 1) / cp;  // pieces per chunk, chunks
+    const size_t cp = chunk / piece, nch = (np + cp - 1) / cp;  // pieces per chunk, chunks
     size_t launched = 0, issued = 0;
     auto rearrange = [&] {  // the next chunk
         const size_t c0 = launched * cp * cells, c1 = std::min<size_t>(Nc, c0 + cp * cells);
-        launch_rows(tmp + (launched & 1) * CHUNK, phi, G, Np, Nc, c0, c1 - c0, st);
+        launch_rows(tmp.p[launched & 1], phi, G, Np, Nc, c0, c1 - c0, st);
         RT_HIP(hipEventRecord(r.chunk_ev[launched & 1], st));
         ++launched;
     };
@@ -260,7 +262,7 @@ void engine_out(Ring& r, double* out, const double* phi, int G, int Np, int Nc, 
             const int s = (int)(issued % slots);
             r.wait_slot(s);
             const size_t n = std::min(cells, (size_t)Nc - issued * cells) * per;
-            RT_HIP(hipMemcpyAsync(r.buf + s * piece, tmp + (c & 1) * CHUNK + (issued - c * cp) * cells * per,
+            RT_HIP(hipMemcpyAsync(r.buf + s * piece, tmp.p[c & 1] + (issued - c * cp) * cells * per,
                                   n * sizeof(double), hipMemcpyDeviceToHost, r.st[issued % STREAMS]));
         }
         RT_HIP(hipStreamSynchronize(r.st[k % STREAMS]));
@@ -274,46 +276,51 @@ void engine_out(Ring& r, double* out, const double* phi, int G, int Np, int Nc, 
 
 }  // namespace
 
-void flux_to_host(double* out, const double* phi, int G, int Np, int Nc, FluxWay way, hipStream_t st) {
+void flux_to_host(double* out, const double* phi, int G, int Np, int Nc, FluxWay way, const FluxScratch& scratch,
+                  hipStream_t st) {
     const size_t per = (size_t)G * Np, total = per * Nc;
     Ring& r = ring();
-    std::unique_lock<std::mutex> lk(r.use);
-    // beside other work one launch for what fits a piece, as each waits its turn
-    const size_t piece = std::max(way == FLUX_ENGINE ? PIECE_MAX : piece_size(total), std::min(per, PIECE_MAX));
+    std::unique_lock<std::mutex> lk(r.use);  // held to the end: the calls on one problem share its scratch
+    // beside other work one launch for what fits a piece, as each waits its turn; chunks where the
+    // scratch holds them
+    const size_t chunk = std::min(CHUNK_MAX, scratch.n);
+    const bool engine = way == FLUX_ENGINE && total > PIECE_MAX && chunk >= std::max(CHUNK_MIN, per);
+    const size_t piece = engine ? std::min(PIECE_MAX, chunk)
+                                : std::max(way == FLUX_ENGINE ? PIECE_MAX : piece_size(total), std::min(per, PIECE_MAX));
     if (way == FLUX_DIRECT || per > piece || !r.ready()) {
         lk.unlock();
         direct_out(out, phi, G, Np, Nc, st);
         return;
     }
-    double* tmp = nullptr;
-    if (way == FLUX_ENGINE && total > piece) try {
-            tmp = (double*)dev_alloc(2 * CHUNK * sizeof(double));
-        } catch (const Error&) {  // no memory for the chunks: the kernels write the ring
-        }
     try {
-        if (tmp) engine_out(r, out, phi, G, Np, Nc, piece, tmp, st);
+        if (engine) engine_out(r, out, phi, G, Np, Nc, piece, scratch, chunk, st);
         else link_out(r, out, phi, G, Np, Nc, piece, st);
     } catch (...) {
         (void)hipStreamSynchronize(st);
         for (auto q : r.st) (void)hipStreamSynchronize(q);
         r.wait_all();
-        dev_free(tmp);
         throw;
     }
-    dev_free(tmp);
 }
 
-void test_flux_out(int way, int G, int Np, int Nc, const double* phi, double* out) {
+void test_flux_out(int way, int G, int Np, int Nc, const double* phi, size_t chunk, double* out) {
     const size_t bytes = (size_t)G * Np * Nc * sizeof(double);
     double* d = (double*)dev_alloc(bytes);
-    try {
-        RT_HIP(hipMemcpy(d, phi, bytes, hipMemcpyHostToDevice));
-        flux_to_host(out, d, G, Np, Nc, (FluxWay)way, nullptr);
-    } catch (...) {
+    FluxScratch s{{nullptr, nullptr}, chunk};
+    auto free_all = [&] {
+        for (double* p : s.p) dev_free(p);
         dev_free(d);
+    };
+    try {
+        if (chunk > 0)
+            for (double*& p : s.p) p = (double*)dev_alloc(chunk * sizeof(double));
+        RT_HIP(hipMemcpy(d, phi, bytes, hipMemcpyHostToDevice));
+        flux_to_host(out, d, G, Np, Nc, (FluxWay)way, s, nullptr);
+    } catch (...) {
+        free_all();
         throw;
     }
-    dev_free(d);
+    free_all();
 }
 
 }  // namespace rt

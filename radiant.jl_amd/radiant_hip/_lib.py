@@ -102,7 +102,7 @@ def lib():
     L.rt_solve_batch.argtypes = [C.c_int32, C.POINTER(PD), C.POINTER(dp), C.POINTER(GS), C.POINTER(SolveInfo)]
     L.rt_problem_kernel_times.argtypes = [H, dp, lp]
     L.rt_test_contraction.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, dp, dp, dp]
-    L.rt_test_flux_out.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32, dp, dp]
+    L.rt_test_flux_out.argtypes = [C.c_int32, C.c_int32, C.c_int32, C.c_int32, dp, C.c_int64, dp]
     L.rt_batch_create.argtypes = [C.c_int32, C.POINTER(PD), C.POINTER(H)]
     L.rt_batch_solve.argtypes = [H, C.POINTER(GS), C.POINTER(SolveInfo)]
     L.rt_batch_get_flux.argtypes = [H, C.c_int32, dp]

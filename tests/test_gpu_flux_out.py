@@ -8,24 +8,29 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 LINK, ENGINE, DIRECT = 0, 1, 2
+FULL = 8 << 20  # doubles of a whole chunk
 
 
 # One small piece (copied by the caller), one cell, some 2 MiB pieces with a ragged end, 50 pieces of
 # 4 MiB in 24 slots and 38 of 8 MiB in 12 (every slot used again), a cell's moments of just under and
 # beyond a piece (the latter without the ring), one value per cell (more cells than a grid's second axis
-# holds tiles); by the copy engines one piece, whole and ragged chunks of eight 8 MiB pieces.
-@pytest.mark.parametrize("way,G,Np,Nc", [
-    (LINK, 3, 5, 7), (LINK, 1, 1, 1), (LINK, 3, 16, 30690), (LINK, 4, 30, 218461), (LINK, 7, 31, 181003),
-    (LINK, 1024, 1023, 3), (LINK, 1024, 1025, 3), (LINK, 1, 1, 2500003),
-    (ENGINE, 3, 5, 7), (ENGINE, 1, 1, (1 << 20) + 1), (ENGINE, 4, 16, 2 * (1 << 17)), (ENGINE, 4, 30, 218461),
-    (ENGINE, 7, 31, 181003), (ENGINE, 1024, 1023, 20), (ENGINE, 1, 1, 9000001),
-    (DIRECT, 3, 5, 7), (DIRECT, 7, 31, 81003), (DIRECT, 1, 1, 4200001)])
-def test_pieces(way, G, Np, Nc):
+# holds tiles); by the copy engines one piece, whole and ragged chunks of eight 8 MiB pieces, and blocks
+# that hold two pieces and a rest, one, less than a whole one, and none.
+@pytest.mark.parametrize("way,G,Np,Nc,chunk", [
+    (LINK, 3, 5, 7, 0), (LINK, 1, 1, 1, 0), (LINK, 3, 16, 30690, 0), (LINK, 4, 30, 218461, 0),
+    (LINK, 7, 31, 181003, 0), (LINK, 1024, 1023, 3, 0), (LINK, 1024, 1025, 3, 0), (LINK, 1, 1, 2500003, 0),
+    (ENGINE, 3, 5, 7, FULL), (ENGINE, 1, 1, (1 << 20) + 1, FULL), (ENGINE, 4, 16, 2 * (1 << 17), FULL),
+    (ENGINE, 4, 30, 218461, FULL), (ENGINE, 7, 31, 181003, FULL + 999), (ENGINE, 1024, 1023, 20, FULL),
+    (ENGINE, 1, 1, 9000001, FULL), (ENGINE, 7, 31, 81003, 2250000), (ENGINE, 7, 31, 81003, 1 << 20),
+    (ENGINE, 7, 31, 81003, 150000), (ENGINE, 7, 31, 31003, 1 << 17), (ENGINE, 7, 31, 31003, (1 << 17) - 1),
+    (ENGINE, 1024, 1023, 20, 1024 * 1023 - 1), (ENGINE, 1024, 1025, 3, FULL), (ENGINE, 7, 31, 31003, 0),
+    (DIRECT, 3, 5, 7, 0), (DIRECT, 7, 31, 81003, 0), (DIRECT, 1, 1, 4200001, 0)])
+def test_pieces(way, G, Np, Nc, chunk):
     from radiant_hip import _lib
     phi = np.arange(G * Np * Nc, dtype=np.float64).reshape(G, Np, Nc)
     out = np.full((Nc, Np, G), np.nan)
-    print(way, G, Np, Nc, phi.nbytes, flush=True)
-    _lib.check(_lib.lib().rt_test_flux_out(way, G, Np, Nc, _lib.ptr(phi), _lib.ptr(out)))
+    print(way, G, Np, Nc, chunk, phi.nbytes, flush=True)
+    _lib.check(_lib.lib().rt_test_flux_out(way, G, Np, Nc, _lib.ptr(phi), chunk, _lib.ptr(out)))
     assert np.array_equal(out.transpose(2, 1, 0), phi)
 
 
